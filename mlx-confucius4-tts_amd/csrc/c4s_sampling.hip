@@ -1257,6 +1257,7 @@ constexpr int kT2MaxV = 1 << 19;    // above: the LDS holds the history bitmap o
 struct T2Sh {
   uint32_t hist[kT2Copies][kT2Buckets];
   uint64_t list[kT2Cap];
+  uint64_t sorted[256];             // the rank sort's result (list itself after the bitonic network)
   double e[kT2Cap];                 // the draw's masses in id order
   uint32_t wsum[NW];
   float wmax[NW];
@@ -1272,21 +1273,33 @@ struct T2Sh {
 
 __host__ __device__ __forceinline__ size_t t2_offset(int V) { return ((size_t)4 * ((V + 31) / 32) + 15) & ~(size_t)15; }
 
-// Descending sort of n <= NT distinct 64-bit keys by rank counting (each key's
-// place is the count of keys above it), through tmp; two barriers.
-__device__ __forceinline__ void rank_sort_desc_u64(uint64_t* buf, uint64_t* tmp, int n) {
-  const int t = threadIdx.x;
-  if (t < n) {
-    const uint64_t mine = buf[t];
-    int r = 0;
-    for (int j = 0; j < n; ++j) r += (buf[j] > mine) ? 1 : 0;
-    tmp[r] = mine;
+constexpr int kRankSortMax = 256;   // above: the bitonic network
+// Descending sort of n <= kRankSortMax distinct 64-bit keys by rank counting
+// (each key's place is the count of keys above it) into `out`; one barrier. The
+// four lanes of a quad share a key and count over every fourth entry each (a
+// thread a key: 3.6k cycles for the 80 entries of a top_k 50 row).
+__device__ __forceinline__ void rank_sort_desc_u64(const uint64_t* buf, uint64_t* out, int n) {
+  static_assert(4 * kRankSortMax == NT, "a quad a key");
+  const int t = threadIdx.x, nS = __builtin_amdgcn_readfirstlane(n), q = t & 3, i = t >> 2;
+  if (__builtin_amdgcn_readfirstlane(i & ~15) < nS) {   // waves whose keys all lie past n
+    const uint64_t mine = buf[min(i, nS - 1)];
+    uint32_t r = 0;
+    int j = 0;
+    for (; j + 16 <= nS; j += 16) {
+      uint64_t o[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o[u] = buf[j + 4 * u + q];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) r += o[u] > mine ? 1u : 0u;
+    }
+    for (; j < nS; j += 4)
+      if (j + q < nS) r += buf[j + q] > mine ? 1u : 0u;
+    r += xor_lane_u32<1>(r);
+    r += xor_lane_u32<2>(r);
+    if (q == 0 && i < nS) out[r] = mine;
   }
   __syncthreads();
-  if (t < n) buf[t] = tmp[t];
-  __syncthreads();
 }
-constexpr int kRankSortMax = 256;   // above: the bitonic network
 
 // In-buffer descending bitonic sort of P (a power of two) 64-bit keys by the
 // NT threads of the workgroup.
@@ -1586,20 +1599,21 @@ __device__ __forceinline__ bool topk_one_read(const RowsArgs& a, const RowCfg& c
   }
 }
 
-// top_k, top_p and the draw on the sorted candidates ts.list[0, ts.n) (every
+// top_k, top_p and the draw on the sorted candidates list[0, ts.n) (every
 // entry at or above the k-th largest value among them); returns true.
 __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const RowCfg& c, const T2Row& src, T2Sh& ts,
-                            uint32_t stat_bits) {
+                            uint64_t* list, uint32_t stat_bits) {
   const int V = c.V, t = threadIdx.x, w = wave_id(), lane = lane_id();
   const float ninf = neg_inf();
   const uint32_t k = (uint32_t)c.k;
   const int n = (int)ts.n;
   // top_k: every entry with the k-th largest value or above survives
-  const uint32_t kkey = (uint32_t)(ts.list[k - 1] >> 32);
+  const uint32_t kkey = (uint32_t)(list[k - 1] >> 32);
   if (w == 0) {
     int ns = (int)k;
-    while (ns < n && (uint32_t)(ts.list[ns] >> 32) >= kkey) ++ns;
-    const float vmax = kfloat((uint32_t)(ts.list[0] >> 32));
+    for (int more = kWave; more == kWave && ns < n; ns += more)   // a run of ties ends the survivors
+      more = __popcll(__ballot(ns + lane < n && (uint32_t)(list[min(ns + lane, n - 1)] >> 32) >= kkey));
+    const float vmax = kfloat((uint32_t)(list[0] >> 32));
     int nkeep = ns, tok = -2;   // -2: not decided here
     uint32_t dex = 0u;
     if (ns <= kWave) {
@@ -1609,7 +1623,7 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
       // sequential replay of lane_draw (the draw), as the candidate-list step
       // does. Survivor j's mass is exp(z_j - vmax), vmax the first survivor's.
       const bool sv = lane < ns;
-      const uint64_t ent = ts.list[sv ? lane : 0];
+      const uint64_t ent = list[sv ? lane : 0];
       const float zs = sv ? kfloat((uint32_t)(ent >> 32)) : ninf;
       const int ids = (int)~(uint32_t)ent;
       const double e = sv ? exp((double)(zs - vmax)) : 0.0;
@@ -1649,7 +1663,7 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
       double total = 0.0;
       for (int base = 0; base < ns; base += kWave) {
         const int j = base + lane;
-        const double e = j < ns ? exp((double)(kfloat((uint32_t)(ts.list[ns - 1 - j] >> 32)) - vmax)) : 0.0;
+        const double e = j < ns ? exp((double)(kfloat((uint32_t)(list[ns - 1 - j] >> 32)) - vmax)) : 0.0;
         total = seq_sum_lanes(total, e, min(kWave, ns - base));
       }
       const double thr = 1.0 - (double)c.p;
@@ -1658,7 +1672,7 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
       bool stop = false;
       for (int base = 0; base < ns && !stop; base += kWave) {
         const int j = base + lane;
-        const double q = j < ns ? exp((double)(kfloat((uint32_t)(ts.list[ns - 1 - j] >> 32)) - vmax)) / total : 0.0;
+        const double q = j < ns ? exp((double)(kfloat((uint32_t)(list[ns - 1 - j] >> 32)) - vmax)) / total : 0.0;
         removed = base + seq_cut_lanes(cum, q, min(kWave, ns - base), thr, stop);
       }
       nkeep = ns - removed;
@@ -1680,7 +1694,7 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
     for (int i = t; i < V; i += NT) mrow[i] = ninf;
     __syncthreads();
     for (int j = t; j < nkeep; j += NT) {   // the row's own value (the key folds -0 onto +0)
-      const int i = (int)~(uint32_t)ts.list[j];
+      const int i = (int)~(uint32_t)list[j];
       mrow[i] = src.z(i, src.xf ? src.xf[i] : __uint_as_float((uint32_t)src.xb[i] << 16));
     }
   }
@@ -1706,23 +1720,28 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
   __syncthreads();
   const int Ps = nkeep <= kRankSortMax ? nkeep : Pk;
   for (int j = t; j < Ps; j += NT) {
-    const uint64_t v = j < nkeep ? ts.list[j] : 0ull;
-    ts.list[j] = j < nkeep ? (((uint64_t)(uint32_t)v << 32) | (v >> 32)) : 0ull;
+    const uint64_t v = j < nkeep ? list[j] : 0ull;
+    list[j] = j < nkeep ? (((uint64_t)(uint32_t)v << 32) | (v >> 32)) : 0ull;
   }
   __syncthreads();
-  if (nkeep <= kRankSortMax) rank_sort_desc_u64(ts.list, reinterpret_cast<uint64_t*>(ts.e), nkeep);
-  else bitonic_desc_u64(ts.list, Pk);
+  if (nkeep <= kRankSortMax) {
+    uint64_t* out = list == ts.list ? ts.sorted : ts.list;
+    rank_sort_desc_u64(list, out, nkeep);
+    list = out;
+  } else {
+    bitonic_desc_u64(list, Pk);
+  }
   C4S_PHASE(6);
   if (w == 0) {
     // text2semantic.cpp:150-165 over the kept entries in id order (the maximum
     // starts from -1e30f; -inf positions add 0)
     float m = -1e30f;
-    for (int j = lane; j < nkeep; j += kWave) m = fmaxf(m, kfloat((uint32_t)ts.list[j]));
+    for (int j = lane; j < nkeep; j += kWave) m = fmaxf(m, kfloat((uint32_t)list[j]));
     m = wave_max_f32(m);
     double total = 0.0;
     for (int base = 0; base < nkeep; base += kWave) {
       const int j = base + lane;
-      const float zj = j < nkeep ? kfloat((uint32_t)ts.list[j]) : ninf;
+      const float zj = j < nkeep ? kfloat((uint32_t)list[j]) : ninf;
       const double e = (j < nkeep && zj != ninf) ? exp((double)(zj - m)) : 0.0;
       if (j < nkeep) ts.e[j] = e;
       total = seq_sum_lanes(total, e, min(kWave, nkeep - base));
@@ -1737,7 +1756,7 @@ __device__ __forceinline__ bool topk_finish(const RowsArgs& a, int row, const Ro
       const double e = j < nkeep ? ts.e[j] : 0.0;
       const int q = seq_find_lanes(acc, e, min(kWave, nkeep - base), r);
       if (q >= 0) {
-        tok = (int)~(uint32_t)(ts.list[base + q] >> 32);
+        tok = (int)~(uint32_t)(list[base + q] >> 32);
         done = true;
       }
     }
@@ -1769,10 +1788,12 @@ __device__ __forceinline__ bool topk_two_pass(const RowsArgs& a, int row, const 
   uint32_t qkey = 0u;
   bool one = src.xf && V <= kOneMaxV && (!c.pen_on || c.pen >= 1.0f) &&
              topk_one_read(a, c, src.xf, src.bitmap, ts, qkey, first);
+  uint64_t* list = ts.list;
   if (one) {
     const int n = (int)ts.n;
     if (n <= kRankSortMax) {
-      rank_sort_desc_u64(ts.list, reinterpret_cast<uint64_t*>(ts.e), n);   // the draw's masses come later
+      rank_sort_desc_u64(ts.list, ts.sorted, n);
+      list = ts.sorted;
     } else {
       int P = 1;
       while (P < n) P <<= 1;
@@ -1782,9 +1803,9 @@ __device__ __forceinline__ bool topk_two_pass(const RowsArgs& a, int row, const 
     }
     C4S_PHASE(4);
     // no value below the bound ties the k-th quotient (the largest of them, divided)
-    if (c.temp_on && !(fkey(kfloat(qkey - 1u) / c.temp) < (uint32_t)(ts.list[k - 1] >> 32))) one = false;
+    if (c.temp_on && !(fkey(kfloat(qkey - 1u) / c.temp) < (uint32_t)(list[k - 1] >> 32))) one = false;
   }
-  if (one) return topk_finish(a, row, c, src, ts, 64u);
+  if (one) return topk_finish(a, row, c, src, ts, list, 64u);
   __syncthreads();   // the work area is free again
   for (int i = t; i < kT2Copies * kT2Buckets; i += NT) (&ts.hist[0][0])[i] = 0u;
   if (t == 0) ts.n = 0u;
@@ -1830,34 +1851,47 @@ __device__ __forceinline__ bool topk_two_pass(const RowsArgs& a, int row, const 
   for (int i = n + t; i < P; i += NT) ts.list[i] = 0ull;
   __syncthreads();
   bitonic_desc_u64(ts.list, P);
-  return topk_finish(a, row, c, src, ts, 0u);
+  return topk_finish(a, row, c, src, ts, ts.list, 0u);
 }
 
-__global__ __launch_bounds__(NT) void k_rows_global(RowsArgs a) {
-  C4S_PHASE(14);
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Scratch sh;
-  const int row = blockIdx.x;
-  const int V = a.vocab;
-  // the row's flags and parameters by scalar loads, all issued before any
-  // waits for them (a byte flag read as its aligned word: flag_byte)
+}  // namespace
+}  // namespace c4s
+
+#include "c4s_big.hpp"
+
+namespace c4s {
+namespace {
+
+// A row's flags, parameters and history offsets by scalar loads, all issued
+// before any waits for them (a byte flag read as its aligned word: flag_byte);
+// false for an inactive row.
+__device__ __forceinline__ bool global_cfg(const RowsArgs& a, int row, RowCfg& c, int64_t& h0, int64_t& h1) {
+  h0 = h1 = 0;
+  if (a.hist_off && !a.hist_bits) {
+    h0 = a.hist_off[row];
+    h1 = a.hist_off[row + 1];
+  }
   const bool act = a.row_active ? flag_byte(a.row_active, row) : true;
   const bool sample = a.do_sample ? flag_byte(a.do_sample, row) : true;
   const float pv = a.pen ? a.pen[row] : 1.0f, tv = a.temp ? a.temp[row] : 1.0f;
   const int32_t kv = a.top_k ? a.top_k[row] : 0, mv = a.min_keep ? a.min_keep[row] : 1;
   const float ppv = a.top_p ? a.top_p[row] : 1.0f;
-  if (!act) {
-    if (threadIdx.x == 0) a.out_tok[row] = -1;
-    return;
-  }
-  const RowCfg c = make_cfg_vals(a.mode, V, pv, tv, kv, ppv, mv, (a.mode & kCustom) || sample);
+  c = make_cfg_vals(a.mode, a.vocab, pv, tv, kv, ppv, mv, (a.mode & kCustom) || sample);
+  if (!c.pen_on) h0 = h1 = 0;
+  return act;
+}
+
+// The general path of one row (the whole workgroup): the top-k reads where
+// they apply, else the multi-pass chain re-reading the row.
+__device__ __forceinline__ void rows_global_row(const RowsArgs& a, int row, const RowCfg& c, int64_t h0, int64_t h1,
+                                                unsigned char* smem, Scratch& sh) {
+  const int V = a.vocab;
   const int64_t roff = (int64_t)row * a.ld;
   // The history's first ids (four a thread), then, for a row that the top-k
   // read takes, that read's first loads: in flight during the set-up (loads
   // complete in issue order, so the ids come first)
   constexpr int kPreIds = 4;
   const bool csr = c.pen_on && !a.hist_bits;
-  const int64_t h0 = csr ? a.hist_off[row] : 0, h1 = csr ? a.hist_off[row + 1] : 0;
   int hid[kPreIds];
   {
     const int nb = (int)min(h1 - h0, (int64_t)NT * kPreIds) * 4;   // the first ids' bytes
@@ -1930,6 +1964,139 @@ __global__ __launch_bounds__(NT) void k_rows_global(RowsArgs a) {
     if (c.draw && a.rng) a.rng[row] = rng;
     join_history(a, row, tok);
   }
+}
+// Whether the top-k read in one pass over the row takes it (fp32, penalty >= 1).
+__device__ __forceinline__ bool one_read_applies(const RowsArgs& a, const RowCfg& c) {
+  return c.draw && c.topk_on && c.k <= kT2MaxK && a.rng && a.dtype == 0 && c.V <= kOneMaxV &&
+         (!c.pen_on || c.pen >= 1.0f);
+}
+
+template <int EPV, bool kPhases>
+__global__ __launch_bounds__(NT) void k_rows_global(RowsArgs a) {
+  C4S_PHASE(14);
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ Scratch sh;
+  const int row = blockIdx.x;
+  RowCfg c;
+  int64_t h0, h1;
+  if (!global_cfg(a, row, c, h0, h1)) {
+    if (threadIdx.x == 0) a.out_tok[row] = -1;
+    return;
+  }
+  if (kPhases && __builtin_expect(!one_read_applies(a, c) && big_covers(a, c), 0)) {
+    if (big_single<EPV>(a, row, c, h0, h1, smem)) return;
+    __syncthreads();
+  }
+  rows_global_row(a, row, c, h0, h1, smem, sh);
+}
+
+constexpr int kBigThreads = 512;   // phases A and B by slices
+
+// Whether a call goes a launch a phase (else one workgroup a row). Both forms,
+// microseconds a call at V = 151936 (10 slices; top_k / nucleus / greedy):
+// fp32, 32 rows 25.6 / 48 / 15.4 against 25.3 / 159 / 37, 48 rows 26.8 / 50 /
+// 16 against 25.4 / 161 / 37, 64 rows 33 / 66 / 20 against 25.7 / 163 / 37:
+// fp32 top-k rows have the one read, so the launches stop paying where their
+// workgroups pass the CUs; bf16, 32 rows 24 / 52 / 15 against 77 / 160 / 35, 256
+// rows 68 / 159 / 40 against 79 / 164 / 36. At V = 20000 (2 slices) the
+// launches cost more than spreading gives: 64 fp32 rows 20 / 35 / 14 against
+// 13 / 45 / 11.
+bool big_by_phase(const RowsArgs& a) {
+  const int nsl = big_slices(a.vocab);
+  return a.dtype == 0 ? nsl >= 8 && (int64_t)nsl * a.n_rows <= 320 : nsl >= 4;
+}
+
+// Workgroup -> (row, slice): consecutive workgroups go to the XCDs in turn, so
+// workgroup 8 i + x takes slices of rows x, x + 8, ...: a row's slices share
+// one XCD's L2, where phase B merges their histograms. The grid is rounded up
+// to whole groups of 8 rows; false past the last row.
+__device__ __forceinline__ bool big_place(const RowsArgs& a, int& row, int& s) {
+  const int nsl = big_slices(a.vocab), i = (int)blockIdx.x >> 3;
+  row = 8 * (i / nsl) + ((int)blockIdx.x & 7);
+  s = i % nsl;
+  return row < a.n_rows;
+}
+
+template <int EPV>
+__global__ __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_big_a(RowsArgs a) {
+  __shared__ BigShA sh;
+  C4S_PHASE(0);
+  int row, s;
+  if (!big_place(a, row, s)) return;
+  const BigGeo g = big_geo(a, row);
+  BigFetch<kSlice / kBigThreads, EPV> f;
+  big_fetch<kSlice / kBigThreads, EPV>(g, s, f);   // in flight while the parameters arrive
+  RowCfg c;
+  int64_t h0, h1;
+  if (!global_cfg(a, row, c, h0, h1) || !big_covers(a, c)) return;
+  const BigHist hs = big_hist<kBigThreads>(a, h0, h1);
+  const int nsl = big_slices(c.V);
+  big_phase_a<kBigThreads, EPV>(a, row, c, g, big_row(c), hs, f, big_ws(a, row, nsl), s, sh);
+}
+
+template <int EPV>
+__global__ __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_big_b(RowsArgs a) {
+  __shared__ BigShB sh;
+  C4S_PHASE(7);
+  int row, s;
+  if (!big_place(a, row, s)) return;
+  const BigGeo g = big_geo(a, row);
+  const int nsl = big_slices(a.vocab);
+  const BigWs ws = big_ws(a, row, nsl);
+  // in issue order: the headers and histograms (of a row that has none, what
+  // its workspace holds), the slice
+  BigMerge<kBigThreads> mf;
+  big_window_fetch<kBigThreads>(ws, nsl, mf);
+  RowCfg c;
+  int64_t h0, h1;
+  if (!global_cfg(a, row, c, h0, h1) || !big_covers(a, c) || c.greedy || c.topk_on) return;
+  BigFetch<kSlice / kBigThreads, EPV> f;
+  big_fetch<kSlice / kBigThreads, EPV>(g, s, f);
+  const BigHist hs = big_hist<kBigThreads>(a, h0, h1);
+  BigWin win;
+  const bool ok = big_window<kBigThreads>(c, ws, nsl, sh, mf, win);
+  if (s == 0 && threadIdx.x == 0) {
+    ws.hdr->wm = win.m;
+    ws.hdr->wxlo = win.xlo;
+    ws.hdr->wxhi = ok ? win.xhi : kBigNB;
+  }
+  if (!ok) return;
+  C4S_PHASE(8);
+  big_phase_b<kBigThreads, EPV>(a, row, c, g, big_row(c), hs, f, ws, s, win, sh);
+}
+
+__global__ __launch_bounds__(NT) void k_big_c(RowsArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ Scratch sh;
+  const int row = blockIdx.x;
+  C4S_PHASE(20);
+  RowCfg c;
+  int64_t h0, h1;
+  if (!global_cfg(a, row, c, h0, h1)) {
+    if (threadIdx.x == 0) a.out_tok[row] = -1;
+    return;
+  }
+  if (big_covers(a, c)) {
+    const int nsl = big_slices(c.V);
+    const BigWs ws = big_ws(a, row, nsl);
+    const BigHist hs = big_hist<NT>(a, h0, c.greedy || c.topk_on ? h0 : h1);
+    BigWin win{};
+    bool ok = true;
+    if (!c.greedy && !c.topk_on) {
+      win.m = ws.hdr->wm;
+      win.fQ = floorf(win.m * kBigScale);
+      win.xlo = ws.hdr->wxlo;
+      win.xhi = ws.hdr->wxhi;
+      ok = win.xhi < kBigNB;
+    }
+    C4S_PHASE(12);
+    if (ok && big_finish<kSlice / kBigThreads>(a, row, c, big_geo(a, row), big_row(c), hs, ws, nsl, win, smem)) {
+      C4S_PHASE(21);
+      return;
+    }
+    __syncthreads();
+  }
+  rows_global_row(a, row, c, h0, h1, smem, sh);
 }
 
 // hist_bits[b] = the ids in [0, V) of row b's CSR history (sampling.cpp:24).
@@ -2034,7 +2201,8 @@ size_t rows_lds_bytes(int V) {
 size_t stream_lds_bytes(int V, int) { return rows_lds_bytes(V); }
 
 size_t rows_global_lds_bytes(int V) {
-  return V <= kT2MaxV ? t2_offset(V) + sizeof(T2Sh) : 4 * (size_t)((V + 31) / 32);
+  const size_t own = V <= kT2MaxV ? t2_offset(V) + sizeof(T2Sh) : 4 * (size_t)((V + 31) / 32);
+  return own > kBigFinishBytes ? own : kBigFinishBytes;
 }
 
 size_t rows_step_lds_bytes(int V) {
@@ -2064,7 +2232,21 @@ hipError_t launch_rows(const RowsArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_rows_lds, dim3(a.n_rows), dim3(NT), lds, s, a);
   } else {
     const size_t lds = rows_global_lds_bytes(a.vocab);
-    hipLaunchKernelGGL(k_rows_global, dim3(a.n_rows), dim3(NT), lds, s, a);
+    if (a.mode == 0u && !a.out_masked && big_by_phase(a)) {
+      const dim3 g(8 * big_slices(a.vocab) * ((a.n_rows + 7) / 8));
+      if (a.dtype == 0) {
+        hipLaunchKernelGGL(k_big_a<4>, g, dim3(kBigThreads), 0, s, a);
+        hipLaunchKernelGGL(k_big_b<4>, g, dim3(kBigThreads), 0, s, a);
+      } else {
+        hipLaunchKernelGGL(k_big_a<8>, g, dim3(kBigThreads), 0, s, a);
+        hipLaunchKernelGGL(k_big_b<8>, g, dim3(kBigThreads), 0, s, a);
+      }
+      hipLaunchKernelGGL(k_big_c, dim3(a.n_rows), dim3(NT), lds, s, a);
+    } else {
+      if (a.mode != 0u || a.out_masked) hipLaunchKernelGGL((k_rows_global<4, false>), dim3(a.n_rows), dim3(NT), lds, s, a);
+      else if (a.dtype == 0) hipLaunchKernelGGL((k_rows_global<4, true>), dim3(a.n_rows), dim3(NT), lds, s, a);
+      else hipLaunchKernelGGL((k_rows_global<8, true>), dim3(a.n_rows), dim3(NT), lds, s, a);
+    }
   }
   return hipGetLastError();
 }
