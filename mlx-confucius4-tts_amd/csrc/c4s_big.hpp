@@ -86,30 +86,6 @@ __device__ __forceinline__ BigWs big_ws(const RowsArgs& a, int row, int nsl) {
   return w;
 }
 
-// exp(t) for t <= 0 (-inf gives 0) to about an ulp: 2^n e^r, |r| <= ln 2 / 2,
-// e^r by its Taylor polynomial of degree 12 (the first term left out is below
-// 2^-52 e^r); rel_eps covers a few ulp.
-__device__ __forceinline__ double exp_neg(double t) {
-  t = fmax(t, -746.0);   // 0 from there on
-  const double n = rint(t * 0x1.71547652b82fep+0);
-  double r = __builtin_fma(n, -0x1.62e42fefa0000p-1, t);   // the high part of ln 2: n times it is exact
-  r = __builtin_fma(n, -0x1.cf79abc9e3b3ap-40, r);
-  double p = 1.0 / 479001600.0;
-  p = __builtin_fma(p, r, 1.0 / 39916800.0);
-  p = __builtin_fma(p, r, 1.0 / 3628800.0);
-  p = __builtin_fma(p, r, 1.0 / 362880.0);
-  p = __builtin_fma(p, r, 1.0 / 40320.0);
-  p = __builtin_fma(p, r, 1.0 / 5040.0);
-  p = __builtin_fma(p, r, 1.0 / 720.0);
-  p = __builtin_fma(p, r, 1.0 / 120.0);
-  p = __builtin_fma(p, r, 1.0 / 24.0);
-  p = __builtin_fma(p, r, 1.0 / 6.0);
-  p = __builtin_fma(p, r, 0.5);
-  p = __builtin_fma(p, r, 1.0);
-  p = __builtin_fma(p, r, 1.0);
-  return ldexp(p, (int)n);
-}
-
 // The row as the slices see it: element position p stands for id p - off, so
 // that 16-byte loads at multiples of 16 bytes are aligned whatever the row's
 // first address.

@@ -193,6 +193,30 @@ __device__ __forceinline__ uint64_t xor_lane_u64(uint64_t v) {
 // One multiply and two conversions instead of the IEEE divide's ten steps.
 __device__ __forceinline__ float div_rcp(float x, double r) { return (float)((double)x * r); }
 
+// exp(t) for t <= 0 (-inf gives 0) to about an ulp: 2^n e^r, |r| <= ln 2 / 2,
+// e^r by its Taylor polynomial of degree 12 (the first term left out is below
+// 2^-52 e^r); rel_eps covers a few ulp.
+__device__ __forceinline__ double exp_neg(double t) {
+  t = fmax(t, -746.0);   // 0 from there on
+  const double n = rint(t * 0x1.71547652b82fep+0);
+  double r = __builtin_fma(n, -0x1.62e42fefa0000p-1, t);   // the high part of ln 2: n times it is exact
+  r = __builtin_fma(n, -0x1.cf79abc9e3b3ap-40, r);
+  double p = 1.0 / 479001600.0;
+  p = __builtin_fma(p, r, 1.0 / 39916800.0);
+  p = __builtin_fma(p, r, 1.0 / 3628800.0);
+  p = __builtin_fma(p, r, 1.0 / 362880.0);
+  p = __builtin_fma(p, r, 1.0 / 40320.0);
+  p = __builtin_fma(p, r, 1.0 / 5040.0);
+  p = __builtin_fma(p, r, 1.0 / 720.0);
+  p = __builtin_fma(p, r, 1.0 / 120.0);
+  p = __builtin_fma(p, r, 1.0 / 24.0);
+  p = __builtin_fma(p, r, 1.0 / 6.0);
+  p = __builtin_fma(p, r, 0.5);
+  p = __builtin_fma(p, r, 1.0);
+  p = __builtin_fma(p, r, 1.0);
+  return ldexp(p, (int)n);
+}
+
 // x_{i+1} = fl(x_i + q) for i < m (q > 0 and x_0 > 0 finite, below 2^53):
 // the final x_m and the number of i <= m with x_i <= thr (a prefix: x does
 // not decrease). Stepping a binade at a time: with x = C ulp (C in [2^52,

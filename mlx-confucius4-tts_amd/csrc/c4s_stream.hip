@@ -30,6 +30,7 @@
 // penalty can raise values (penalty < 1) take the exact chain every step.
 
 #include "c4s_list.hpp"
+#include "c4s_nucleus.hpp"
 
 namespace c4s {
 namespace {
@@ -2462,12 +2463,19 @@ __global__ __launch_bounds__(NT) void k_stream_chain(StreamArgs a, StreamWs w) {
 // gathers the drawn ids' raw values from the step's row in HBM, and wave 0
 // gathers, for each decided token, its raw values in the next 64 steps, so
 // that the check reads LDS only. A step no summary path settles stops every
-// wave for the exact chain on the row read into LDS.
+// wave for an exact step on the row read into LDS: nucleus_lds, else the
+// multi-pass chain. On a row whose nucleus is wider than the list at most steps
+// (top_p 0.9 above a temperature of about 1.17 on the 8194-id rows) such steps
+// follow each other, and the waves stay for a run of them: 64 rows x 1000 steps
+// with one such row 54-56 ms on the chain, 33-35 with nucleus_lds, 19-21 with
+// the runs and the row's loads in flight together (about 19 us a step, bound by
+// one row's dependent passes on six waves).
 
 constexpr int kSpecND = 5;                 // decider waves
 constexpr int NTS = (kSpecND + 1) * kWave;
 constexpr int kSpecGv = 1024;              // ids a call can draw (its steps at most)
 constexpr int kRing = 16;                  // per-token value rows kept by wave 0
+constexpr int kExactRun = 31;              // exact steps in a row without asking the deciders
 constexpr int kSpecVW = 3;                 // the checking wave: alone on its SIMD (waves go to SIMDs in turn)
 constexpr int kHist = 8;                   // steps of tokens the checking wave keeps in registers
 static_assert(kHist >= kSpecND, "history covers the steps a decision can lag");
@@ -2517,6 +2525,8 @@ struct SpecCtl {
   int tok;
   uint64_t rng;
   uint32_t acc[4];
+  uint64_t rrng;   // RNG state of step rstep, where the deciders resume after an exact step
+  int rstep;
 };
 
 // Drawn set of one decision: ids whose drawn index is below nF; raw values of
@@ -2550,7 +2560,8 @@ __host__ __device__ inline SpecLayout spec_layout(int V) {
   L.o_cs = al16(L.o_cd + 8 * (size_t)kMaxChunks);
   L.stride = al16(L.o_cs + sizeof(SpecCS));
   size_t dec = (size_t)kSpecND * L.stride;
-  const size_t rowb = al16(4 * ((size_t)vpad(V) + 4));   // the exact chain's row over the deciders' areas
+  // the exact step's row and masses over the deciders' areas
+  const size_t rowb = al16(4 * ((size_t)vpad(V) + 4)) + nucleus_bytes<kSpecND + 1>(V);
   L.total = L.dec + (dec > rowb ? dec : rowb);
   return L;
 }
@@ -2762,7 +2773,16 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
     __syncthreads();
     float* X = reinterpret_cast<float*>(smem + L.dec);
     const float* src = rowp(hq);
-    for (int i = t; i < V; i += NTS) X[i] = src[i];
+    // kRowLoads of a thread's loads in flight at once
+    constexpr int kRowLoads = 11;
+    for (int i0 = t; i0 < V; i0 += NTS * kRowLoads) {
+      float xr[kRowLoads];
+#pragma unroll
+      for (int j = 0; j < kRowLoads; ++j) xr[j] = src[min(i0 + NTS * j, V - 1)];
+#pragma unroll
+      for (int j = 0; j < kRowLoads; ++j)
+        if (i0 + NTS * j < V) X[i0 + NTS * j] = xr[j];
+    }
     __syncthreads();
     if (c.pen_on) {   // H0 and the stream's ids are disjoint: each id once
       penalise_chunk<NTS>(X, bmH0, V, c.pen);
@@ -2771,7 +2791,11 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
     __syncthreads();
     uint64_t r = ctl.rng;
     LdsRowNC srow{X, V, 0u, false, w.sortbuf + (int64_t)row * w.sort_stride, (uint32_t)(w.sort_stride * 4)};
-    const int tok = run_chain(srow, xs, c, r, nullptr, xs.step_stats);
+    int tok = 0;
+    if (!nucleus_lds<kSpecND + 1>(X, c, smem + L.dec + al16(4 * ((size_t)vpad(V) + 4)), r, tok, xs.step_stats)) {
+      __syncthreads();
+      tok = run_chain(srow, xs, c, r, nullptr, xs.step_stats);
+    }
     __syncthreads();
     if (t == 0) {
       ctl.tok = tok;
@@ -2786,7 +2810,8 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
     int n = ctl.snap & 0xFFFF;
     uint64_t rng = rng0;
     uint32_t acc[4] = {ctl.acc[0], ctl.acc[1], ctl.acc[2], ctl.acc[3]};
-    bool stopped = false, bad = ctl.err != 0, expired = false;
+    bool stopped = false, bad = ctl.err != 0, expired = false, run_on = false;
+    int last_exact = -2, exact_run = 0;
     const float rpen = 1.0f / c.pen;
     const double rtemp = 1.0 / (double)c.temp;
     // the last kHist steps: lane (step % kHist) holds the step, its token and
@@ -2923,20 +2948,54 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
       }
       C4S_SPEC_T(4);
       if (exact) {
-        // every wave stops (the deciders' areas hold the row), then resumes at q + 1
-        if (lane == 0) {
-          ctl.rng = rng;
+        // every wave stops (the deciders' areas hold the row), then resumes at
+        // q + 1, or, on a row where steps that only the exact chain settles
+        // follow each other (a nucleus wider than the list at every step), stays
+        // for a run of them: twice as many each time the step after a run is
+        // not settled either
+        int run = q == last_exact + 1 ? exact_run : 0;
+        exact_run = min(2 * run + 1, kExactRun);
+        for (;;) {
+          if (lane == 0) {
+            ctl.rng = rng;
+            lgkm_wait();
+            vstore(&ctl.halt, q);
+          }
+          if (run_on) __syncthreads();   // the deciders enter the next exact step
+          exact_all(q);
+          tokq = ctl.tok;
+          if (lane == 0) {
+            const uint32_t* stp = xs.step_stats;
+            acc[0] |= stp[0];
+            acc[1] += 1u;
+            acc[2] += stp[2];
+            acc[3] += stp[3];
+          }
+          run_on = run > 0 && q + 1 < s_end && tokq != a.stop_token && n < kSpecGv;
+          if (!run_on) break;
+          // the step is done as below, without a ring row: the decisions after
+          // the run know this id
+          --run;
+          if (lane == 0) tout[q - s_first] = (int16_t)tokq;
+          rng = ctl.rng;
+          const bool fr = c.pen_on && tokq >= 0 && tokq < V && !bit_of(bmH0, tokq) && didx[tokq] == 0xFFFFu;
+          if (fr) {
+            if (lane == 0) {
+              tokl[n] = tokq;
+              tstep[n] = (uint16_t)q;
+              didx[tokq] = (uint16_t)n;
+              lds_or(&bmN[tokq >> 5], 1u << (tokq & 31));
+            }
+            ++n;
+          }
+          ++q;
           lgkm_wait();
-          vstore(&ctl.halt, q);
+          if (lane == 0) vstore(&ctl.snap, (q << 16) | n);
         }
-        exact_all(q);
-        tokq = ctl.tok;
+        last_exact = q;
         if (lane == 0) {
-          const uint32_t* stp = xs.step_stats;
-          acc[0] |= stp[0];
-          acc[1] += 1u;
-          acc[2] += stp[2];
-          acc[3] += stp[3];
+          ctl.rstep = q + 1;
+          ctl.rrng = ctl.rng;
           for (int i = 0; i < kSpecND; ++i) recs[i].tag = -1;
         }
         // ring rows of dropped decisions (steps after q) are stale
@@ -3023,14 +3082,10 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
   } else {
     // ---- deciders ----
     const int k = wv < kSpecVW ? wv : wv - 1;
-    auto start_at = [&](int from, int& q, uint64_t& rq) __attribute__((always_inline)) {
-      q = from + (((k - (from - s_first)) % kSpecND) + kSpecND) % kSpecND;
-      rq = rng0;
-      for (int i = s_first; i < q; ++i) rq = xorshift64(rq);
-    };
-    int q;
-    uint64_t rq;
-    start_at(s_first, q, rq);
+    auto first_of = [&](int from) { return from + (((k - (from - s_first)) % kSpecND) + kSpecND) % kSpecND; };
+    int q = first_of(s_first);
+    uint64_t rq = rng0;
+    for (int i = s_first; i < q; ++i) rq = xorshift64(rq);
     SpecCS& cs = dcs(k);
     uint64_t* sw = dsum(k);
     float* gv = dgv(k);
@@ -3057,8 +3112,14 @@ __global__ __launch_bounds__(NTS) void k_stream_spec(StreamArgs a, StreamWs w) {
       if (halted) {
         exact_all(vload(&ctl.halt));
         __syncthreads();   // the checking wave has moved the frontier past the exact step
-        start_at(vload(&ctl.snap) >> 16, q, rq);
-        if (lane == 0) cs.gen = 0u;
+        if (vload(&ctl.halt) < 0) {   // not in a run of exact steps: resume from the new frontier
+          // (rstep and rrng change only while every wave is in an exact step)
+          const int from = ctl.rstep;
+          q = first_of(from);
+          rq = ctl.rrng;
+          for (int i = from; i < q; ++i) rq = xorshift64(rq);
+          if (lane == 0) cs.gen = 0u;
+        }
         continue;
       }
       C4S_SPEC_T(1);
