@@ -427,6 +427,193 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   }
 }
 
+// ---- more than 64 rows -------------------------------------------------------------------
+//
+// k_lmhead's tile (32 columns, 64 rows) converts every weight again for each 64
+// rows and feeds each MFMA pair from one LDS read of x: 777 x 1280 x 8194 took
+// 100 us, 164 TFLOP/s. Here a workgroup owns 128 rows and BN columns, each of
+// its four waves 64 x BN / 2 of them, and the weights of a chunk of 64 inputs
+// are converted once into LDS as the hi and lo parts of W gamma (the same split
+// and sums as k_lmhead: G, c, d and the row statistics in fp32). 8-bit codes
+// are taken to scale q + offset in fp32 first, so that no per-group partial
+// products are needed. Loads run one chunk ahead in registers; two workgroups
+// share a CU, so one converts while the other multiplies. 777 rows: 61 us bf16,
+// 68 fp32, 65 8-bit (k_lmhead 100, 121, 133); a thread's weights as 32 inputs of
+// one column (64 bytes a lane: eight lanes' loads on one line before) 64 / 104 /
+// 65, and gamma and beta loaded by the threads that convert 72 / 102 / 75.
+constexpr int kWdThreads = 256;
+constexpr int kWdM = 128;                  // rows of a workgroup
+constexpr int kWdK = 64;                   // inputs of a chunk
+constexpr int kWdPitch = kWdK * 2 + 16;    // bytes of a staged row (+16: conflict-free reads)
+
+template <int WK, int BN>
+__global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_lmhead_wide(LmHeadArgs a) {
+  constexpr int NB = BN / 32;                       // 16-column blocks of a wave
+  constexpr int kRows = kWdThreads * 8 / kWdK;      // rows (columns) that the threads' pieces of 8 inputs cover
+  constexpr int kXp = kWdM / kRows, kWp = BN / kRows;   // pieces of x and of the weights a thread stages
+  constexpr bool kQ = WK == kLmW_Q8;
+  __shared__ __align__(16) unsigned char xs[kWdM * kWdPitch], wh[BN * kWdPitch], wl[BN * kWdPitch];
+  __shared__ __align__(16) float gb[2][2][kWdK];   // by buffer: gamma, beta of a chunk
+  __shared__ float st1[kWdM], st2[kWdM], rmu[kWdM], rinv[kWdM], ccol[BN], dcol[BN];
+  const int D = a.D, V = a.V, M = a.M;
+  const int n0 = blockIdx.x * BN, m0 = blockIdx.y * kWdM;
+  const int t = threadIdx.x, w = wave_id(), l = lane_id(), r = l & 15, g = l >> 4;
+  const int wm = (w & 1) * 64, wn = (w >> 1) * (BN / 2);   // the wave's rows and columns
+  const int nch = (D + kWdK - 1) / kWdK;
+  f32x4 acc[4][NB], sto[2], stg[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) sto[i] = stg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+  // staging: piece j is row (column) kRows j + t / 8, inputs 8 (t % 8) .. + 7 of
+  // the chunk: eight threads read one row's 128 bytes (bf16), and every piece of
+  // a thread has the same inputs, so gamma and beta are read once a chunk
+  const int pr = t / 8, pk = (t % 8) * 8;
+  WRaw<WK> wr[kWp];
+  float qs[kQ ? kWp : 1], qb[kQ ? kWp : 1];
+  uint4 xv[kXp];
+  float cp[kWp], dp[kWp];
+#pragma unroll
+  for (int j = 0; j < kWp; ++j) cp[j] = dp[j] = 0.f;
+  // gamma (threads 0 .. 15) and beta (16 .. 31), four inputs each, in LDS a chunk ahead
+  const bool gb_t = t < 2 * (kWdK / 4);
+  const int gb_a = t / (kWdK / 4), gb_o = (t % (kWdK / 4)) * 4;
+  float4 gv = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto gb_fetch = [&](int ch) __attribute__((always_inline)) {
+    const int k = ch * kWdK + gb_o;
+    if (gb_t) gv = *reinterpret_cast<const float4*>((gb_a ? a.beta : a.gamma) + (k < D ? k : 0));
+  };
+  auto fetch = [&](int ch) __attribute__((always_inline)) {   // past D: in bounds, not used
+    const int kx = ch * kWdK + pk, k = kx < D ? kx : 0;
+#pragma unroll
+    for (int j = 0; j < kWp; ++j) {
+      const int64_t col = min(n0 + kRows * j + pr, V - 1);
+      wr[j].load(a.weight, col * D + k);
+      if constexpr (kQ) {
+        const int64_t q = col * (D / a.group) + k / a.group;
+        qs[j] = a.wscale[q];
+        qb[j] = a.wbias[q];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kXp; ++j)
+      xv[j] = *reinterpret_cast<const uint4*>(a.hidden + (int64_t)min(m0 + kRows * j + pr, M - 1) * D + k);
+  };
+  gb_fetch(0);
+  if (gb_t) *reinterpret_cast<float4*>(&gb[0][gb_a][gb_o]) = gv;
+  gb_fetch(1);
+  fetch(0);
+  for (int ch = 0; ch < nch; ++ch) {
+    __syncthreads();   // every wave is done with the last chunk
+    if (gb_t) *reinterpret_cast<float4*>(&gb[(ch + 1) & 1][gb_a][gb_o]) = gv;
+    gb_fetch(ch + 2);
+    const bool in = ch * kWdK + pk < D;   // D is a multiple of 32
+#pragma unroll
+    for (int j = 0; j < kXp; ++j)
+      *reinterpret_cast<uint4*>(&xs[(kRows * j + pr) * kWdPitch + pk * 2]) = in ? xv[j] : make_uint4(0u, 0u, 0u, 0u);
+    {
+      const float4* gp = reinterpret_cast<const float4*>(&gb[ch & 1][0][pk]);
+      const float4* bp = reinterpret_cast<const float4*>(&gb[ch & 1][1][pk]);
+      const float4 g0 = gp[0], g1 = gp[1], b0 = bp[0], b1 = bp[1];
+      const float gm[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      const float bt[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+      for (int j = 0; j < kWp; ++j) {
+        float wv[8], wg[8], c1 = 0.f, d1 = 0.f;
+        wr[j].get(wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (kQ) wv[e] = __builtin_fmaf(qs[j], wv[e], qb[j]);
+          wv[e] = in ? wv[e] : 0.f;
+          wg[e] = wv[e] * gm[e];
+          c1 += wg[e];
+          d1 = __builtin_fmaf(wv[e], bt[e], d1);
+        }
+        cp[j] += c1;
+        dp[j] += d1;
+        uint4 hi, lo;
+        split8(wg, hi, lo);
+        *reinterpret_cast<uint4*>(&wh[(kRows * j + pr) * kWdPitch + pk * 2]) = hi;
+        *reinterpret_cast<uint4*>(&wl[(kRows * j + pr) * kWdPitch + pk * 2]) = lo;
+      }
+    }
+    if (ch + 1 < nch) fetch(ch + 1);   // in flight during the products
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < kWdK / 32; ++ks) {
+      const int ko = ks * 64 + g * 16;   // bytes: 32 inputs a step, 8 a lane group
+      uint4 xa[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xa[i] = *reinterpret_cast<const uint4*>(&xs[(wm + 16 * i + r) * kWdPitch + ko]);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const uint4 bh = *reinterpret_cast<const uint4*>(&wh[(wn + 16 * j + r) * kWdPitch + ko]);
+        const uint4 bl = *reinterpret_cast<const uint4*>(&wl[(wn + 16 * j + r) * kWdPitch + ko]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mfma_bf16(xa[i], bh, acc[i][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mfma_bf16(xa[i], bl, acc[i][j]);
+      }
+      // the row statistics, two of the four row blocks by each of the two waves that hold them
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint4 xb = (w >> 1) ? xa[2 + i] : xa[i];
+        sto[i] = mfma_bf16(xb, ones, sto[i]);
+        stg[i] = mfma_bf16(xb, xb, stg[i]);
+      }
+    }
+  }
+  // 16x16 accumulator layout: lane l holds rows 4 (l / 16) + i, column l % 16
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int row = wm + 16 * (2 * (w >> 1) + b);
+    if (r == 0)   // every column of the ones product holds the row sums
+#pragma unroll
+      for (int i = 0; i < 4; ++i) st1[row + 4 * g + i] = sto[b][i];
+    if ((r >> 2) == g) {   // the Gram diagonal: row r at column r
+      const int i = r & 3;
+      st2[row + r] = i == 0 ? stg[b][0] : (i == 1 ? stg[b][1] : (i == 2 ? stg[b][2] : stg[b][3]));
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kWp; ++j) {   // eight threads hold a column's inputs
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      cp[j] += __shfl_xor(cp[j], o, kWave);
+      dp[j] += __shfl_xor(dp[j], o, kWave);
+    }
+    if (t % 8 == 0) {
+      const int cl = kRows * j + pr;
+      ccol[cl] = cp[j];
+      dcol[cl] = dp[j] + a.bias[min(n0 + cl, V - 1)];
+    }
+  }
+  __syncthreads();
+  if (t < kWdM) {
+    const double invD = 1.0 / (double)D;
+    const double mu = (double)st1[t] * invD;
+    rmu[t] = (float)mu;
+    rinv[t] = (float)(1.0 / sqrt(fmax((double)st2[t] * invD - mu * mu, 0.0) + (double)a.eps));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int cl = wn + 16 * j + r, n = n0 + cl;
+    const float cc = ccol[cl], dd = dcol[cl];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = wm + 16 * i + 4 * g + e, m = m0 + row;
+        if (n < V && m < M)
+          a.logits[(int64_t)m * a.ld_out + n] = __builtin_fmaf(rinv[row], __builtin_fmaf(-rmu[row], cc, acc[i][j][e]), dd);
+      }
+  }
+}
+
 // HBM probes: each workgroup streams one contiguous span with four independent
 // 16-byte non-temporal loads per thread in flight.
 constexpr int kProbeThreads = 256;
@@ -474,7 +661,31 @@ static hipError_t launch_k(const LmHeadArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// 64 columns a workgroup until 128 would fill the chip's CUs once.
+// k_lmhead up to kWideRows rows. Both sides, microseconds at D = 1280, V = 8194
+// (bf16 / fp32 / 8-bit): 128 rows 27.1 / 30.1 / 32.1 there, 29.0 / 29.1 / 31.0 here;
+// 256 rows 40.4 / 47.4 / 51.1 there, 38.0 / 38.2 / 39.9 here (rows up to 256 cost
+// the same here, each 64 rows a pass there).
+constexpr int kWideRows = 192;
+template <int WK>
+static hipError_t launch_wide(const LmHeadArgs& a, hipStream_t s) {
+  const int mt = (a.M + kWdM - 1) / kWdM;
+  if ((int64_t)mt * ((a.V + 127) / 128) >= 256)
+    hipLaunchKernelGGL((k_lmhead_wide<WK, 128>), dim3((a.V + 127) / 128, mt), dim3(kWdThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_lmhead_wide<WK, 64>), dim3((a.V + 63) / 64, mt), dim3(kWdThreads), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_lmhead(const LmHeadArgs& a, hipStream_t s) {
+  if (a.M > kWideRows) {
+    switch (a.wkind) {
+      case kLmW_BF16: return launch_wide<kLmW_BF16>(a, s);
+      case kLmW_F32: return launch_wide<kLmW_F32>(a, s);
+      case kLmW_Q8: return launch_wide<kLmW_Q8>(a, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   switch (a.wkind) {
     case kLmW_BF16: return launch_k<kLmW_BF16, 1>(a, s);
     case kLmW_F32: return launch_k<kLmW_F32, 1>(a, s);

@@ -1,0 +1,38 @@
+"""LM head of more rows than its small tile takes, at the edges of its tiles (128 rows, 64 or 128
+columns, chunks of 64 inputs), for the three weight kinds, against the float64
+oracle; the tolerance and its derivation are test_gpu_lmhead's (the same split
+of the weights, the same sums)."""
+import numpy as np
+import pytest
+
+import c4s_workloads as W
+from gpu_util import dev
+from test_gpu_lmhead import ATOL, _weights
+
+pytestmark = pytest.mark.gpu
+
+CASES = [("bf16", 193, 32, 1, 32, 0.0), ("bf16", 255, 96, 63, 32, 0.0), ("bf16", 256, 64, 64, 32, 0.0),
+         ("bf16", 257, 160, 65, 32, 4.0), ("bf16", 192, 160, 65, 32, 0.0), ("bf16", 300, 1280, 8194, 64, 0.0), ("bf16", 777, 1280, 5000, 64, 0.0),
+         ("f32", 193, 96, 129, 32, 0.0), ("f32", 200, 2080, 127, 32, 4.0), ("f32", 520, 256, 8194, 64, 0.0),
+         ("q8", 194, 32, 40, 32, 0.0), ("q8", 230, 192, 65, 64, 0.0), ("q8", 257, 256, 130, 128, 4.0),
+         ("q8", 600, 1280, 8194, 64, 0.0), ("q8", 1000, 96, 4100, 32, 0.0)]
+
+
+@pytest.mark.parametrize("kind,M,D,V,group,shift", CASES)
+def test_lmhead_many_rows(orc, gpu_ctx, kind, M, D, V, group, shift):
+    import torch
+    head, _ = W.lmhead(seed=M + D, M=M, D=D, V=V)
+    if shift:
+        head.hidden = W.f32_to_bf16_bits(W.bf16_bits_to_f32(head.hidden) + np.float32(shift))
+    wdev, quant, worc, kw = _weights(kind, head, M + D + 1, group)
+    ld = V + 3   # rows of the output at every alignment; the columns past V stay as they are
+    logits = torch.full((M, ld), 7.0, dtype=torch.float32, device="cuda")
+    gpu_ctx.lmhead(dev(head.hidden, torch), dev(head.gamma, torch), dev(head.beta, torch), wdev,
+                   dev(head.bias, torch), logits, quant=quant)
+    torch.cuda.synchronize()
+    got = logits.cpu().numpy()
+    assert (got[:, V:] == 7.0).all()
+    want = orc.ln_lmhead(head.hidden, head.gamma, head.beta, worc, head.bias, n_threads=16, **kw)
+    err = np.abs(got[:, :V].astype(np.float64) - want)
+    print(f"{kind} M={M} D={D} V={V}: max abs err {err.max():.3e}  max |logit| {np.abs(want).max():.3f}", flush=True)
+    assert np.all(err <= ATOL)
