@@ -20,7 +20,6 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kTileM = 64;
 constexpr int kTileN = 32;
 
 // ---- LayerNorm folded into the GEMM (one kernel) -------------------------------------
@@ -44,7 +43,8 @@ constexpr int kTileN = 32;
 // sum_k x^2 as the diagonal of the 16x16 Gram block x x^T (bf16 products are
 // exact in fp32).
 //
-// A workgroup owns 32 columns (vocabulary entries) and 64 rows. K goes in
+// A workgroup owns 32 columns (vocabulary entries) and 64 rows (16 or 32 when
+// there are no more). K goes in
 // chunks of eight steps of 32 (256 inputs): the workgroup stages the chunk's
 // rows of x in LDS with 16-byte loads that cover whole cache lines (32 KB, two
 // buffers), and wave w takes the chunk's steps w and w + 4. The first two
@@ -65,12 +65,16 @@ constexpr int kLmWaves = kLmThreads / kWave;
 constexpr int kWaveSteps = 2;                                     // steps a wave takes per chunk
 constexpr int kChunkK = kLmWaves * kWaveSteps * 32;               // inputs per chunk
 constexpr int kXPitch = kChunkK * 2 + 16;                         // bytes per staged row (+16: conflict-free reads)
-constexpr int kXLoads = kTileM * kChunkK * 2 / 16 / kLmThreads;   // 16-byte loads per thread per chunk
 constexpr int kRowPieces = kChunkK / 8;                           // 16-byte pieces per staged row
-constexpr size_t kXBytes = (size_t)kTileM * kXPitch;
-constexpr int kRedPitch = kTileM + 4;                             // floats per column of a partial tile (+4: conflict-free)
-constexpr size_t kRedBytes = (size_t)kLmWaves * kTileN * kRedPitch * 4;
-static_assert(kRedBytes <= 2 * kXBytes, "the partial sums fit over the staging buffers");
+// MT: 16-row blocks of the tile.
+template <int MT> struct LmTile {
+  static constexpr int kM = 16 * MT;
+  static constexpr int kXLoads = kM * kChunkK * 2 / 16 / kLmThreads;   // 16-byte loads per thread per chunk
+  static constexpr size_t kXBytes = (size_t)kM * kXPitch;
+  static constexpr int kRedPitch = kM + 4;                        // floats per column of a partial tile (+4: conflict-free)
+  static constexpr size_t kRedBytes = (size_t)kLmWaves * kTileN * kRedPitch * 4;
+  static_assert(kRedBytes <= 2 * kXBytes, "the partial sums fit over the staging buffers");
+};
 
 // Two floats to two bf16, round to nearest even (v_cvt_pk_bf16_f32); the
 // low halfword holds the first.
@@ -134,16 +138,19 @@ template <> struct WRaw<kLmW_Q8> {
 };
 
 // WK: weight kind; SPU: k-steps of 32 per scale group (1 unless 8-bit).
-template <int WK, int SPU>
+template <int WK, int SPU, int MT>
 __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_lmhead(LmHeadArgs a) {
   constexpr bool kQ = WK == kLmW_Q8;
+  constexpr int kTileM = LmTile<MT>::kM, kXLoads = LmTile<MT>::kXLoads, kRedPitch = LmTile<MT>::kRedPitch;
+  constexpr size_t kXBytes = LmTile<MT>::kXBytes;
   constexpr bool kCdMfma = WK == kLmW_BF16;   // c and d on the matrix engine (the weights are bf16-exact)
   // chunks whose weights a wave keeps in flight (kWaveSteps steps each). Loads
   // complete in issue order, so a chunk's rows of x, issued two chunks ahead,
   // wait behind every weight load issued before them: a window of two chunks
   // (refilled per chunk) instead of the whole of K for bf16 weights took
-  // 64 x 1280 x 8194 from 15.7 to 13.8 us.
-  constexpr int kWin = WK == kLmW_F32 ? 2 : (WK == kLmW_Q8 ? (SPU > 1 ? 2 : 3) : 2);
+  // 64 x 1280 x 8194 from 15.7 to 13.8 us; 1 row, fp32: one chunk 11.45, two 11.6,
+  // all five 13.3 us.
+  constexpr int kWin = MT < 4 ? (kQ ? 2 : 1) : WK == kLmW_F32 ? 2 : (WK == kLmW_Q8 ? (SPU > 1 ? 2 : 3) : 2);
   __shared__ __align__(16) unsigned char xs[2 * kXBytes];
   __shared__ __align__(16) float gbs[2][2][kChunkK];   // by buffer: gamma, beta of the chunk
   // by buffer: gamma hi, gamma lo, beta hi, beta lo as bf16 (rows 0-3 of an MFMA
@@ -160,9 +167,9 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   const int r = l & 15, g = l >> 4;
   const int nsteps = D / 32, nchunks = (nsteps + kLmWaves * kWaveSteps - 1) / (kLmWaves * kWaveSteps);
   // per row block: the two column blocks, then the ones and the Gram products
-  f32x4 acc[4][4];
+  f32x4 acc[MT][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float cp[2] = {0.f, 0.f}, dp[2] = {0.f, 0.f};   // fp32 and 8-bit weights: this lane's parts of c and d
@@ -294,7 +301,7 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
             }
             const unsigned char* xb = &xs[(ch & 1) * kXBytes + kc * 2];
 #pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
               const uint4 xa = *reinterpret_cast<const uint4*>(xb + (mt * 16 + r) * kXPitch);
 #pragma unroll
               for (int nt = 0; nt < 2; ++nt) {
@@ -316,7 +323,7 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   // (the last barrier: every wave is done with the staging buffers)
   // 16x16 accumulator layout: lane l holds rows 4*(l/16)+i, column l%16.
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+  for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt)   // rows 4g .. 4g + 3 of column r: one 16-byte store
       *reinterpret_cast<f32x4*>(&red[w][nt * 16 + r][mt * 16 + 4 * g]) = acc[mt][nt];
@@ -615,8 +622,13 @@ __global__ __launch_bounds__(kProbeThreads) void k_hbm_read(const f32x4* src, fl
 
 template <int WK, int SPU>
 static hipError_t launch_k(const LmHeadArgs& a, hipStream_t s) {
-  const dim3 grid((a.V + kTileN - 1) / kTileN, (a.M + kTileM - 1) / kTileM);
-  hipLaunchKernelGGL((k_lmhead<WK, SPU>), grid, dim3(kLmThreads), 0, s, a);
+  const int mt = (a.M + 63) / 64;
+  const dim3 grid((a.V + kTileN - 1) / kTileN, mt);
+  // A tile of the rows there are: 64 staged and multiplied for one row took
+  // 14.7 us (fp32; bf16 13.1, 8-bit 15.0 for 16 rows) against 11.5 (9.7, 11.6).
+  if (a.M <= 16) hipLaunchKernelGGL((k_lmhead<WK, SPU, 1>), grid, dim3(kLmThreads), 0, s, a);
+  else if (a.M <= 32) hipLaunchKernelGGL((k_lmhead<WK, SPU, 2>), grid, dim3(kLmThreads), 0, s, a);
+  else hipLaunchKernelGGL((k_lmhead<WK, SPU, 4>), grid, dim3(kLmThreads), 0, s, a);
   return hipGetLastError();
 }
 

@@ -1,6 +1,6 @@
-"""LM head of more rows than its small tile takes, at the edges of its tiles (128 rows, 64 or 128
-columns, chunks of 64 inputs), for the three weight kinds, against the float64
-oracle; the tolerance and its derivation are test_gpu_lmhead's (the same split
+"""LM head at the edges of its tiles' row counts (16, 32, 64 and, past 192, 128
+rows with 64 or 128 columns and chunks of 64 inputs), for the three weight kinds,
+against the float64 oracle; the tolerance and its derivation are test_gpu_lmhead's (the same split
 of the weights, the same sums)."""
 import numpy as np
 import pytest
@@ -11,7 +11,10 @@ from test_gpu_lmhead import ATOL, _weights
 
 pytestmark = pytest.mark.gpu
 
-CASES = [("bf16", 193, 32, 1, 32, 0.0), ("bf16", 255, 96, 63, 32, 0.0), ("bf16", 256, 64, 64, 32, 0.0),
+CASES = [("bf16", 1, 1280, 8194, 64, 0.0), ("f32", 1, 320, 33, 32, 4.0), ("q8", 16, 288, 1000, 32, 0.0),
+         ("bf16", 17, 32, 47, 32, 0.0), ("f32", 32, 1280, 500, 32, 0.0), ("q8", 31, 1280, 300, 128, 4.0),
+         ("bf16", 33, 96, 31, 32, 0.0), ("q8", 192, 64, 100, 64, 0.0),
+         ("bf16", 193, 32, 1, 32, 0.0), ("bf16", 255, 96, 63, 32, 0.0), ("bf16", 256, 64, 64, 32, 0.0),
          ("bf16", 257, 160, 65, 32, 4.0), ("bf16", 192, 160, 65, 32, 0.0), ("bf16", 300, 1280, 8194, 64, 0.0), ("bf16", 777, 1280, 5000, 64, 0.0),
          ("f32", 193, 96, 129, 32, 0.0), ("f32", 200, 2080, 127, 32, 4.0), ("f32", 520, 256, 8194, 64, 0.0),
          ("q8", 194, 32, 40, 32, 0.0), ("q8", 230, 192, 65, 64, 0.0), ("q8", 257, 256, 130, 128, 4.0),
