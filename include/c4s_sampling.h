@@ -28,6 +28,12 @@
  *     captured into a graph a workspace never grows (C4S_EINVAL): make one call
  *     of the same shape outside the capture first. Once a captured call used a
  *     workspace, a later growth keeps the old buffer alive until c4s_destroy.
+ *     Rows with vocab > 12288 have a workspace per stream (for up to eight
+ *     streams; a further one waits for the device and takes over the one used
+ *     longest ago), so such calls of one context may be in flight on several
+ *     streams. A graph's replays use the workspace its capture took (its
+ *     stream's, or another stream's that is large enough): the caller orders
+ *     them with other large-vocabulary calls that may share it.
  *   - Input contract: logits are finite or -inf (no +inf/NaN), temperature is
  *     1, <= 0, or keeps logits/temperature finite.
  *   - top_p tie order: when the nucleus cut falls inside a group of equal

@@ -15,12 +15,26 @@
 #include "../../include/c4s_sampling.h"
 #include "c4s_internal.h"
 
+// Workspace of the large-vocabulary rows of one stream.
+struct RowsWs {
+  hipStream_t stream = nullptr;
+  void* p = nullptr;
+  size_t bytes = 0;
+  uint64_t used = 0;   // tick of its last call
+};
+
 struct c4s_ctx {
   int device = 0;
   std::string err;
   hipStream_t host_stream = nullptr;  // used by the synchronous host helpers
-  void* ws = nullptr;                 // large-vocab exact-pass key buffers
+  void* ws = nullptr;                 // stream: exact steps' key buffers
   size_t ws_bytes = 0;
+  // Large-vocabulary rows (slices, lists, exact-pass keys): one per stream that
+  // issues such calls, so that calls on several streams do not share one.
+  static constexpr int kRowsWs = 8;
+  RowsWs rows_ws[kRowsWs];
+  int n_rows_ws = 0;
+  uint64_t rows_tick = 0;
   void* logits_ws = nullptr;          // LM head + sample: logits when the caller gives none
   size_t logits_bytes = 0;
   // host-helper staging: pinned host memory that the device maps
@@ -219,20 +233,55 @@ c4s::RowsArgs to_args(const c4s_rows* r) {
   return a;
 }
 
-// The sort workspace of vocabularies the step cannot stage in LDS.
-int rows_workspace(c4s_ctx* ctx, const c4s_rows* r, hipStream_t s) {
+// The workspace of vocabularies the step cannot stage in LDS, for a call queued
+// on `s` (*out: null below that size). A captured call takes its stream's, or
+// another stream's that is large enough (a graph's replays are ordered by the
+// caller), and never allocates. Past kRowsWs streams the one used longest ago
+// is handed on once the device is idle.
+int rows_workspace(c4s_ctx* ctx, const c4s_rows* r, hipStream_t s, void** out) {
+  *out = nullptr;
   if (r->vocab <= c4s::kLdsVocabMax) return C4S_OK;
-  const size_t per_row = pow2_at_least((size_t)r->vocab) * sizeof(uint32_t);
-  return ensure(ctx, &ctx->ws, &ctx->ws_bytes, per_row * (size_t)r->n_rows, "sort workspace", s);
+  const size_t need = pow2_at_least((size_t)r->vocab) * sizeof(uint32_t) * (size_t)r->n_rows;
+  RowsWs* w = nullptr;
+  for (int i = 0; i < ctx->n_rows_ws; ++i)
+    if (ctx->rows_ws[i].stream == s) w = &ctx->rows_ws[i];
+  if (is_capturing(s)) {
+    for (int i = 0; i < ctx->n_rows_ws && (!w || w->bytes < need); ++i)
+      if (ctx->rows_ws[i].bytes >= need) w = &ctx->rows_ws[i];
+    if (!w || w->bytes < need)
+      return fail(ctx, C4S_EINVAL, "sort workspace: the workspace would grow during graph capture; make one call of "
+                                   "this shape (or larger) outside the capture first");
+    ctx->graph_used = true;
+  } else {
+    if (!w && ctx->n_rows_ws < c4s_ctx::kRowsWs) {
+      w = &ctx->rows_ws[ctx->n_rows_ws++];
+      w->stream = s;
+    } else if (!w) {
+      w = &ctx->rows_ws[0];
+      for (RowsWs& o : ctx->rows_ws)
+        if (o.used < w->used) w = &o;
+      const hipError_t e = hipDeviceSynchronize();
+      if (e != hipSuccess) return hip_fail(ctx, e, "sort workspace");
+      w->stream = s;
+    }
+    if (w->bytes < need) {
+      const int rc = ensure(ctx, &w->p, &w->bytes, need, "sort workspace", s);
+      if (rc) return rc;
+    }
+  }
+  w->used = ++ctx->rows_tick;
+  *out = w->p;
+  return C4S_OK;
 }
 
 int launch_rows_checked(c4s_ctx* ctx, const c4s_rows* r, hipStream_t s) {
   c4s::RowsArgs a = to_args(r);
   if (r->vocab > c4s::kLdsVocabMax) {
     const size_t per_row = pow2_at_least((size_t)r->vocab) * sizeof(uint32_t);
-    int rc = rows_workspace(ctx, r, s);
+    void* ws = nullptr;
+    int rc = rows_workspace(ctx, r, s, &ws);
     if (rc) return rc;
-    a.sort_ws = static_cast<uint32_t*>(ctx->ws);
+    a.sort_ws = static_cast<uint32_t*>(ws);
     a.sort_ws_stride = (int64_t)(per_row / sizeof(uint32_t));
   }
   hipError_t e = c4s::launch_rows(a, s);
@@ -312,6 +361,8 @@ int c4s_destroy(c4s_ctx* ctx) {
     if (st) (void)hipStreamSynchronize(st);
   for (void* p : {ctx->ws, ctx->logits_ws, ctx->sum_ws, ctx->state_ws, ctx->segres})
     if (p) (void)hipFree(p);
+  for (const RowsWs& w : ctx->rows_ws)
+    if (w.p) (void)hipFree(w.p);
   for (void* p : ctx->retired) (void)hipFree(p);
   if (ctx->host_stream) (void)hipStreamDestroy(ctx->host_stream);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
@@ -692,7 +743,8 @@ int c4s_lmhead_sample(c4s_ctx* ctx, const c4s_head* head, const c4s_rows* rows, 
     logits = static_cast<float*>(ctx->logits_ws);
     r.logits = logits;
   }
-  rc = rows_workspace(ctx, &r, s);
+  void* ws = nullptr;
+  rc = rows_workspace(ctx, &r, s, &ws);
   if (rc) return rc;
   rc = lmhead_launch(ctx, head, logits, r.ld, s);
   if (rc) return rc;

@@ -109,3 +109,35 @@ def test_history_set(orc, gpu_ctx, rows, V):
         for i, k in enumerate(want.tolist()):
             if k != V - 1:
                 hist[i].append(k)
+
+
+@pytest.mark.parametrize("n_streams", [2, 10])
+def test_streams_of_one_context(gpu_ctx, n_streams):
+    """Calls of one context on several streams at once (more of them than the
+    context keeps workspaces for, too), of different shapes: the same tokens and
+    states as one call after the other."""
+    import torch
+    bs = [_batch(31 + i, 16, [131073, 151936, 140001][i % 3]) for i in range(n_streams)]
+    dv = [{k: dev(getattr(b, k), torch) for k in ("logits", "hist_ids", "hist_off", "temp", "top_k", "top_p", "pen",
+                                                  "do_sample")} for b in bs]
+
+    def run(streams):
+        rngs = [dev(b.rng, torch) for b in bs]
+        toks = [[torch.empty(16, dtype=torch.int32, device="cuda") for _ in range(4)] for _ in bs]
+        torch.cuda.synchronize()
+        for step in range(4):
+            for i, d in enumerate(dv):
+                gpu_ctx.sample_rows(d["logits"], d["hist_ids"], d["hist_off"], d["temp"], d["top_k"], d["top_p"],
+                                    d["pen"], rngs[i], toks[i][step], do_sample=d["do_sample"], stream=streams[i])
+                if streams[0] is None:
+                    torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        return [[t.cpu().numpy() for t in ts] for ts in toks], [r.cpu().numpy() for r in rngs]
+
+    want = run([None] * n_streams)
+    got = run([torch.cuda.Stream() for _ in bs])
+    for w, g in zip(want[0], got[0]):
+        for a, b in zip(w, g):
+            assert np.array_equal(a, b)
+    for a, b in zip(want[1], got[1]):
+        assert np.array_equal(a, b)
