@@ -1,4 +1,4 @@
-// The one-pass step (k_rows_step, sampled_step) in the form for more rows
+// The one-pass step (k_rows_step, sampled_step) in the form for many more rows
 // than CUs: two workgroups share a CU.
 //
 // The step is a chain of short barrier-separated phases; one workgroup of eight
@@ -9,10 +9,10 @@
 // in registers over the calls (the unrolled passes at 128 registers spilled 44
 // of them: 46 us for 1000 nucleus rows against 47.7 for the other form and 38.4
 // rolled), and the fp32 masses are taken again instead of kept in LDS. One
-// workgroup alone takes longer this way, so up to as many rows as CUs keep the
-// other form. 1000 rows of 8194 ids, microseconds a call (other form / this):
-// assorted 44.6 / 34.8, pipeline defaults 35.7 / 23.4, nucleus bf16 47.7 / 38.4,
-// greedy 24.9 / 16.2, 1024 rows of ties 138.4 / 105.4; 300 rows assorted 21.4 / 20.9.
+// workgroup alone takes longer this way, so kManyRows is where the line lies.
+// 1000 rows of 8194 ids, microseconds a call (other form / this): assorted
+// 44.6 / 34.8, pipeline defaults 35.7 / 23.4, nucleus bf16 47.7 / 38.4,
+// greedy 24.9 / 16.2, 1024 rows of ties 138.4 / 105.4.
 //
 // The decisions, margins and fallbacks are sampled_step's.
 
@@ -22,6 +22,12 @@ namespace c4s {
 namespace {
 
 constexpr int kManyU = 6;   // a thread's ids read together
+// Up to two rounds of one workgroup a CU, and a little over, a row that falls to
+// its exact replay sets the call, and it takes longer beside another: bf16 rows
+// with ties, 309 rows of 5132 ids 143 / 184 us and of 2500 ids 93 / 108, 513 rows
+// of 5132 ids 181 / 187. Above, the rounds saved are worth more: 700 rows of 5132
+// ids 263 / 203, of 2500 ids 164 / 123, of 8194 ids 108 / 90.
+constexpr int kManyRows = 576;
 
 // draw_finish, with the kept masses taken again from the row in LDS.
 __device__ __forceinline__ void draw_finish_many(const StepIO& io, const RowCfg& c, const KeptRule& kr, int lo, int n,
@@ -513,7 +519,7 @@ __device__ __forceinline__ void chain_fallback_global(const StepIO& io, const Ro
   }
 }
 
-// k_rows_step for more rows than CUs.
+// k_rows_step for many more rows than CUs.
 template <int PT>
 __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_rows_step_many(RowsArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -685,13 +691,13 @@ size_t many_lds_bytes(int V) { return kStepWorkBytes + 4 * ((size_t)vpad(V) + 4)
 
 }  // namespace
 
-// More rows than CUs, two of them in a CU's LDS (static part included: up to
+// More than 2.25 rows a CU (kManyRows), two of them in a CU's LDS (static part included: up to
 // about 9200 ids), the exact top_p's keys (a power of two) within one row's.
 bool rows_step_many_fits(const RowsArgs& a) {
   constexpr size_t kStatic = sizeof(StepScratch) + sizeof(StepSh) + sizeof(StepRowSh) + 256;
   size_t keys = 1;
   while (keys < (size_t)a.vocab) keys <<= 1;
-  return a.n_rows > 256 && 2 * (many_lds_bytes(a.vocab) + kStatic) <= 160 * 1024 &&
+  return a.n_rows > kManyRows && 2 * (many_lds_bytes(a.vocab) + kStatic) <= 160 * 1024 &&
          kStepWorkBytes + 4 * (size_t)vpad(a.vocab) >= 4 * keys;
 }
 

@@ -1,4 +1,4 @@
-"""More rows than CUs: the one-pass step in the form that shares a CU, against
+"""Many more rows than CUs: the one-pass step in the form that shares a CU, against
 the oracle bit for bit -- vocabularies at the sizes where the ids a thread owns
 change and on both sides of the largest one that fits, every row kind, and the
 rows that one pass leaves to the chain."""
@@ -26,7 +26,7 @@ def _rows(seed, n, V, sigma):
 @pytest.mark.parametrize("masked", [True, False])
 @pytest.mark.parametrize("V", [1, 3, 65, 513, 4608, 4609, 8194, 8704, 9000, 9300])
 def test_vocab_sizes(orc, gpu_ctx, V, masked):
-    b, mk = _rows(V, 300, V, 2.0)
+    b, mk = _rows(V, 600, V, 2.0)
     compare_with_oracle(orc, gpu_ctx, b, min_keep=mk, masked=masked)
 
 
@@ -36,7 +36,7 @@ def test_kinds(orc, gpu_ctx, sigma, dtype):
     """Flat rows (the refined boundary), peaked ones, and rows wider than the
     masses' exponent range; then rows for the chain: all -inf, one finite value,
     below the draw's floor, every value equal, two values."""
-    V, n = 8194, 520
+    V, n = 8194, 600
     b, mk = _rows(5, n, V, sigma)
     # p = 0 with min_tokens_to_keep 0 removes every id unless the last sum of the
     # quotients rounds above 1, which the chain behind both forms of the step does
@@ -64,7 +64,7 @@ def test_kinds(orc, gpu_ctx, sigma, dtype):
 
 def test_history_set(orc, gpu_ctx):
     import torch
-    V, n = 4097, 400
+    V, n = 4097, 600
     b, _ = _rows(9, n, V, 2.0)
     hist = [b.hist_ids[b.hist_off[i]:b.hist_off[i + 1]].tolist() for i in range(n)]
     bits = torch.zeros((n, (V + 31) // 32), dtype=torch.int32, device="cuda")
