@@ -265,7 +265,8 @@ struct BigShA {
 };
 
 // Bin of hist (2048 bins, from the top) holding the m-th largest counted key,
-// and the count above it; false (uniform) when fewer were counted.
+// and the count above it; false (uniform) when fewer were counted. Either way a
+// barrier has passed since the last read of red, so the caller may write it.
 template <int NTH>
 __device__ __forceinline__ bool big_pick(const uint32_t* hist, uint32_t* red, uint32_t* out, uint32_t m, uint32_t& bin,
                                          uint32_t& above) {
@@ -284,7 +285,10 @@ __device__ __forceinline__ bool big_pick(const uint32_t* hist, uint32_t* red, ui
     ex += i < wave_id() ? x : 0u;
     total += x;
   }
-  if (total < m) return false;
+  if (total < m) {
+    __syncthreads();
+    return false;
+  }
   if (ex < m && ex + loc >= m) {
     uint32_t run = ex;
 #pragma unroll

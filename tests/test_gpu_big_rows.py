@@ -85,6 +85,32 @@ def test_boundaries(orc, gpu_ctx, rows, V):
     assert (tok[act == 0] == -1).all()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,V", [(16, 16385), (16, 65573), (16, 131073), (260, 16385), (30, 151600)])
+def test_topk_few_in_a_slice(orc, gpu_ctx, rows, V, dtype):
+    """top_k rows whose slices hold fewer than k + 1 values: a last slice of one
+    to a few dozen ids, slices of -inf but for none, one, k or k + 1 values."""
+    b = _batch(V + rows, rows, V, hist=50)
+    k = np.array([1, 2, 7, 49, 50, 63, 64, 120], np.int32)[np.arange(rows) % 8]
+    b.top_k, b.do_sample = k, np.ones(rows, np.uint8)
+    b.top_p = np.where(np.arange(rows) % 3 == 0, 1.0, 0.9).astype(np.float32)
+    b.pen = np.where(np.arange(rows) % 2 == 0, 1.2, 0.8).astype(np.float32)   # below 1: not the one read
+    g = np.random.default_rng(rows)
+    for r in range(rows):
+        for s in range(0, V, 16384):
+            m = min(16384, V - s)
+            few = [m, 0, 1, int(k[r]), int(k[r]) + 1][(r + s // 16384) % 5]
+            if few < m:
+                keep = g.choice(m, few, replace=False)
+                part = b.logits[r, s:s + m][keep]
+                b.logits[r, s:s + m] = -np.inf
+                b.logits[r, s + keep] = part
+    b.logits[:, 5] = 1.0   # no row without a finite value
+    if dtype == "bf16":
+        b.logits = W.f32_to_bf16_bits(b.logits)
+    compare_with_oracle(orc, gpu_ctx, b, masked=False)
+
+
 @pytest.mark.parametrize("rows,V", [(9, 131077), (200, 20011)])
 def test_history_set(orc, gpu_ctx, rows, V):
     """The history kept as a set: three steps, each token joining it."""
