@@ -436,8 +436,10 @@ __device__ __forceinline__ void big_phase_a(const RowsArgs& a, int row, const Ro
   for (int i = 0; i < NTH / kWave; ++i) ms = fmaxf(ms, sh.wf[i]);
   if (t == 0) h->ms = ms;
   C4S_PHASE(25);
-  // dense rows (p >= 1) have no boundary to find
-  if (!(c.p < 1.0f) || !(fabsf(ms) < 0x1p18f)) return;   // uniform
+  // Dense rows (p >= 1) have no boundary to find. The bound on ms takes in every
+  // slice that big_window counts: a row's maximum below 2^18 in magnitude and
+  // slices within 32 of it (the grid's differences are exact up to 2^19).
+  if (!(c.p < 1.0f) || !(fabsf(ms) < 0x1p19f)) return;   // uniform
   const float fqs = floorf(ms * kBigScale);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
@@ -786,6 +788,9 @@ __device__ __forceinline__ bool big_phase_c(const RowsArgs& a, int row, const Ro
     // entry j is removed iff the mass at or below it in ascending order,
     // M = S - (mass above it), is <= thr S (sampling.cpp:60-65)
     const double A = thr * S, mg = rel_eps(c.V) * S, B = S - A;
+    // what lies above X is kept unseen: only where its exact mass falls short of
+    // the boundary, whatever the histograms said
+    if (!(Ma < B - 2.0 * mg)) return false;   // uniform
     // where the kept set ends among the sub-buckets, from mass m0 and n0 entries before them
     auto sub_scan = [&](double m0, uint32_t n0) {
       if (w == 0) {

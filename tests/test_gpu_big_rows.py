@@ -111,6 +111,29 @@ def test_topk_few_in_a_slice(orc, gpu_ctx, rows, V, dtype):
     compare_with_oracle(orc, gpu_ctx, b, masked=False)
 
 
+@pytest.mark.parametrize("rows,V", [(9, 140000), (260, 40000)])
+def test_maxima_about_the_grids_end(orc, gpu_ctx, rows, V):
+    """Nucleus rows with slice maxima on both sides of -2^18 and 2^18, where the
+    histograms' grid ends for a row's maximum; each after a call whose rows leave
+    other histograms in the same workspace."""
+    b = _batch(5, rows, V, sigma=1.0, hist=50)
+    b.do_sample[:], b.top_k[:], b.temp[:], b.pen[:] = 1, 0, 1.0, 1.0
+    b.top_p = np.choose(np.arange(rows) % 3, [0.5, 0.8, 0.95]).astype(np.float32)
+    x = np.clip(b.logits, -8.0, 2.0)
+    s = np.arange(V) // 16384
+    x_far = x - 8.0 - 2.0 * ((s[None, :] + np.arange(rows)[:, None]) % 4)
+    at = (np.arange(rows) * 7919) % V
+    for end, top in ((-262144.0, -262143.0), (262144.0, 262143.0)):
+        b.logits = np.full_like(x, -10.0)   # its masses at lower grid places than the next rows'
+        compare_with_oracle(orc, gpu_ctx, b, masked=False)
+        y = (x_far + end).astype(np.float32)
+        y[np.arange(rows), at] = np.float32(top)   # the row's maximum
+        b.logits = y
+        _, st = compare_with_oracle(orc, gpu_ctx, b, masked=False)
+        if end < 0:   # settled by the phases, on this row's own histograms
+            assert np.count_nonzero(st[:, 0] & 16) >= rows - 2 - rows // 20, st[:, 0].tolist()
+
+
 @pytest.mark.parametrize("rows,V", [(9, 131077), (200, 20011)])
 def test_history_set(orc, gpu_ctx, rows, V):
     """The history kept as a set: three steps, each token joining it."""
