@@ -393,20 +393,31 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   }
 }
 
-// ---- more than 64 rows -------------------------------------------------------------------
+// ---- many rows ---------------------------------------------------------------------------
 //
 // k_lmhead's tile (32 columns, 64 rows) converts every weight again for each 64
 // rows and feeds each MFMA pair from one LDS read of x: 777 x 1280 x 8194 took
 // 100 us, 164 TFLOP/s. Here a workgroup owns 128 rows and BN columns, each of
 // its four waves 64 x BN / 2 of them, and the weights of a chunk of 64 inputs
-// are converted once into LDS as the hi and lo parts of W gamma (the same split
-// and sums as k_lmhead: G, c, d and the row statistics in fp32). 8-bit codes
-// are taken to scale q + offset in fp32 first, so that no per-group partial
-// products are needed. Loads run one chunk ahead in registers; two workgroups
-// share a CU, so one converts while the other multiplies. 777 rows: 61 us bf16,
-// 68 fp32, 65 8-bit (k_lmhead 100, 121, 133); a thread's weights as 32 inputs of
-// one column (64 bytes a lane: eight lanes' loads on one line before) 64 / 104 /
-// 65, and gamma and beta loaded by the threads that convert 72 / 102 / 75.
+// are converted once into LDS as the hi and lo parts of W gamma (k_lmhead's
+// split). 8-bit codes are taken to scale q + offset in fp32 first, so that no
+// per-group partial products are needed. Loads run one chunk ahead in registers;
+// two workgroups share a CU, so one converts while the other multiplies. 777
+// rows: 59 us bf16, 64 fp32, 63 8-bit (k_lmhead 100, 121, 133); a thread's
+// weights as 32 inputs of one column (64 bytes a lane: eight lanes' loads on one
+// line before) 64 / 104 / 65, and gamma and beta loaded by the threads that
+// convert 72 / 102 / 75.
+//
+// The sums that a row's offset cancels against are kept short, as k_lmhead's
+// are: the row statistics as fp32 sums over a quarter of D, c and d over an
+// eighth, joined in double. As one fp32 sum over D each (and d + bias in fp32)
+// rows offset by 16 sigma were off by 4.8e-5 (D = 1280) and 6.1e-5 (D = 4096)
+// of the logits, now 3.9e-5 and 4.6e-5; k_lmhead 3.9e-5 and 4.5e-5. A quarter
+// ends where no load of a chunk is in flight: at the end of the loop body
+// instead, 73 us bf16; as a loop around the chunks, 60. G's own sum runs over
+// all of D in the accumulators (k_lmhead: four, joined in fp32), which is 0.5%
+// of the error at D = 1280 and 2% at 4096; a second set of accumulators beside
+// the first does not fit the registers (74 us).
 constexpr int kWdThreads = 256;
 constexpr int kWdM = 128;                  // rows of a workgroup
 constexpr int kWdK = 64;                   // inputs of a chunk
@@ -420,7 +431,8 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
   constexpr bool kQ = WK == kLmW_Q8;
   __shared__ __align__(16) unsigned char xs[kWdM * kWdPitch], wh[BN * kWdPitch], wl[BN * kWdPitch];
   __shared__ __align__(16) float gb[2][2][kWdK];   // by buffer: gamma, beta of a chunk
-  __shared__ float st1[kWdM], st2[kWdM], rmu[kWdM], rinv[kWdM], ccol[BN], dcol[BN];
+  __shared__ float st1[4][kWdM], st2[4][kWdM];   // by quarter of D: a row's sums of x and of x^2
+  __shared__ float rmu[kWdM], rinv[kWdM], ccol[BN], dcol[BN];
   const int D = a.D, V = a.V, M = a.M;
   const int n0 = blockIdx.x * BN, m0 = blockIdx.y * kWdM;
   const int t = threadIdx.x, w = wave_id(), l = lane_id(), r = l & 15, g = l >> 4;
@@ -452,21 +464,48 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
     const int k = ch * kWdK + gb_o;
     if (gb_t) gv = *reinterpret_cast<const float4*>((gb_a ? a.beta : a.gamma) + (k < D ? k : 0));
   };
+  // offsets from the workgroup's first column and row, which are uniform: 32 bits each
+  constexpr int kWs = kQ ? 1 : WK == kLmW_F32 ? 4 : 2;   // bytes of a stored weight
+  const unsigned char* wbase = static_cast<const unsigned char*>(a.weight) + (int64_t)n0 * D * kWs;
+  const uint16_t* xbase = a.hidden + (int64_t)m0 * D;
+  const int ngr = kQ ? D / a.group : 0;
+  const float* sbase = kQ ? a.wscale + (int64_t)n0 * ngr : nullptr;
+  const float* bbase = kQ ? a.wbias + (int64_t)n0 * ngr : nullptr;
   auto fetch = [&](int ch) __attribute__((always_inline)) {   // past D: in bounds, not used
     const int kx = ch * kWdK + pk, k = kx < D ? kx : 0;
 #pragma unroll
     for (int j = 0; j < kWp; ++j) {
-      const int64_t col = min(n0 + kRows * j + pr, V - 1);
-      wr[j].load(a.weight, col * D + k);
+      const int col = min(kRows * j + pr, V - 1 - n0);
+      wr[j].load(wbase, (uint32_t)(col * D + k));
       if constexpr (kQ) {
-        const int64_t q = col * (D / a.group) + k / a.group;
-        qs[j] = a.wscale[q];
-        qb[j] = a.wbias[q];
+        const uint32_t q = (uint32_t)(col * ngr + k / a.group);
+        qs[j] = sbase[q];
+        qb[j] = bbase[q];
       }
     }
 #pragma unroll
     for (int j = 0; j < kXp; ++j)
-      xv[j] = *reinterpret_cast<const uint4*>(a.hidden + (int64_t)min(m0 + kRows * j + pr, M - 1) * D + k);
+      xv[j] = *reinterpret_cast<const uint4*>(xbase + (uint32_t)(min(kRows * j + pr, M - 1 - m0) * D + k));
+  };
+  // The row statistics so far to their quarter's place, and started again. 16x16
+  // accumulator layout: lane l holds rows 4 (l / 16) + i, column l % 16; row r of a
+  // block goes by the lane that holds it at column r: the Gram diagonal, and every
+  // column of the ones product holds the row sums.
+  const int nq = (nch + 3) / 4;   // chunks of a quarter
+  int q = 0;
+  auto keep = [&]() __attribute__((always_inline)) {
+    if ((r >> 2) == g) {
+      const int i = r & 3;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int row = wm + 16 * (2 * (w >> 1) + b) + r;
+        st1[q][row] = i == 0 ? sto[b][0] : (i == 1 ? sto[b][1] : (i == 2 ? sto[b][2] : sto[b][3]));
+        st2[q][row] = i == 0 ? stg[b][0] : (i == 1 ? stg[b][1] : (i == 2 ? stg[b][2] : stg[b][3]));
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) sto[b] = stg[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    ++q;
   };
   gb_fetch(0);
   if (gb_t) *reinterpret_cast<float4*>(&gb[0][gb_a][gb_o]) = gv;
@@ -506,6 +545,7 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
         *reinterpret_cast<uint4*>(&wl[(kRows * j + pr) * kWdPitch + pk * 2]) = lo;
       }
     }
+    if (ch == nq * (q + 1)) keep();   // with no load of a chunk in flight
     if (ch + 1 < nch) fetch(ch + 1);   // in flight during the products
     __syncthreads();
 #pragma unroll
@@ -532,37 +572,32 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
       }
     }
   }
-  // 16x16 accumulator layout: lane l holds rows 4 (l / 16) + i, column l % 16
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int row = wm + 16 * (2 * (w >> 1) + b);
-    if (r == 0)   // every column of the ones product holds the row sums
-#pragma unroll
-      for (int i = 0; i < 4; ++i) st1[row + 4 * g + i] = sto[b][i];
-    if ((r >> 2) == g) {   // the Gram diagonal: row r at column r
-      const int i = r & 3;
-      st2[row + r] = i == 0 ? stg[b][0] : (i == 1 ? stg[b][1] : (i == 2 ? stg[b][2] : stg[b][3]));
-    }
-  }
+  keep();
 #pragma unroll
   for (int j = 0; j < kWp; ++j) {   // eight threads hold a column's inputs
+    double cc = (double)cp[j], dd = (double)dp[j];
 #pragma unroll
     for (int o = 1; o < 8; o <<= 1) {
-      cp[j] += __shfl_xor(cp[j], o, kWave);
-      dp[j] += __shfl_xor(dp[j], o, kWave);
+      cc += __shfl_xor(cc, o, kWave);
+      dd += __shfl_xor(dd, o, kWave);
     }
     if (t % 8 == 0) {
       const int cl = kRows * j + pr;
-      ccol[cl] = cp[j];
-      dcol[cl] = dp[j] + a.bias[min(n0 + cl, V - 1)];
+      ccol[cl] = (float)cc;
+      dcol[cl] = (float)(dd + (double)a.bias[min(n0 + cl, V - 1)]);
     }
   }
   __syncthreads();
   if (t < kWdM) {
     const double invD = 1.0 / (double)D;
-    const double mu = (double)st1[t] * invD;
+    double S1 = 0.0, S2 = 0.0;
+    for (int i = 0; i < q; ++i) {   // the quarters that D has
+      S1 += (double)st1[i][t];
+      S2 += (double)st2[i][t];
+    }
+    const double mu = S1 * invD;
     rmu[t] = (float)mu;
-    rinv[t] = (float)(1.0 / sqrt(fmax((double)st2[t] * invD - mu * mu, 0.0) + (double)a.eps));
+    rinv[t] = (float)(1.0 / sqrt(fmax(S2 * invD - mu * mu, 0.0) + (double)a.eps));
   }
   __syncthreads();
 #pragma unroll

@@ -39,3 +39,39 @@ def test_lmhead_many_rows(orc, gpu_ctx, kind, M, D, V, group, shift):
     err = np.abs(got[:, :V].astype(np.float64) - want)
     print(f"{kind} M={M} D={D} V={V}: max abs err {err.max():.3e}  max |logit| {np.abs(want).max():.3f}", flush=True)
     assert np.all(err <= ATOL)
+
+
+@pytest.mark.parametrize("kind,D,sigmas", [("f32", 1280, 64.0), ("q8", 1280, 64.0), ("f32", 4096, 16.0), ("q8", 4096, 16.0)])
+def test_offset_rows(gpu_ctx, kind, D, sigmas):
+    """Rows far from mean 0, whose offset cancels between the products, the row
+    statistics and c: a call of many rows is as close to 64 bits as a call of few.
+    Both take sums of the same lengths, so their errors are draws of one spread;
+    of a 2-norm over 192 rows that is off by 1 / sqrt(2 x 192) = 5%: three times
+    that. With each sum as one fp32 sum over D the ratios were 2.5 and 1.36
+    (1.04 and 1.02 with them in parts joined in double)."""
+    import torch
+    V, n = 4200, 192
+    g = torch.Generator(device="cuda")
+    g.manual_seed(D)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")   # noqa: E731
+    x = (rand(200, D) + sigmas).to(torch.bfloat16)
+    gamma, beta, bias, w = 1.0 + 0.02 * rand(D), 0.02 * rand(D), 0.02 * rand(V), 0.02 * rand(V, D)
+    quant, wd = None, w.double()
+    if kind == "q8":
+        grp = w.view(V, D // 64, 64)
+        lo, scale = grp.amin(dim=2), (grp.amax(dim=2) - grp.amin(dim=2)) / 255.0
+        q = torch.clamp(torch.round((grp - lo[..., None]) / scale[..., None]), 0, 255)
+        wd = (q.double() * scale.double()[..., None] + lo.double()[..., None]).view(V, D)
+        w, quant = q.to(torch.uint8).view(V, D), (scale.contiguous(), lo.contiguous(), 64)
+    y = x.double() - x.double().mean(dim=1, keepdim=True)
+    y = y / (y.square().mean(dim=1, keepdim=True) + 1e-5).sqrt() * gamma.double() + beta.double()
+    want = (y @ wd.t() + bias.double())[:n]
+
+    def error(rows):
+        logits = torch.empty((rows, V), device="cuda")
+        gpu_ctx.lmhead(x[:rows].contiguous(), gamma, beta, w, bias, logits, quant=quant)
+        return float((logits[:n].double() - want).norm() / want.norm())
+
+    few, many = error(n), error(200)
+    print(f"{kind} D={D} offset {sigmas} sigma: {few:.3e} of {n} rows, {many:.3e} of 200", flush=True)
+    assert many <= 1.15 * few
