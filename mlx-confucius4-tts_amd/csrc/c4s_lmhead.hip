@@ -1,6 +1,6 @@
 // LM head ahead of the sampler: final LayerNorm + semantic_head linear
 // (src/t2s/text2semantic.cpp:118-121 -> src/nn/nn.cpp:73-83 and :11-16) in one
-// kernel, k_lmhead, for weights in bf16, fp32 (the reference's own dtype: its
+// kernel, k_lmhead or (many rows) k_lmhead_wide, for weights in bf16, fp32 (the reference's own dtype: its
 // .npy weights load as float32, include/c4tts/npy.h:202-206) or 8-bit affine
 // groups (the quantized_matmul layout the reference uses for its projections,
 // src/t2s/gpt2.cpp:49-62: w = scale * q + bias per group of `group`
@@ -8,6 +8,8 @@
 // k_hbm_probe: streaming copy / read kernels for the achievable-bandwidth line.
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "c4s_device.hpp"
 #include "c4s_internal.h"
@@ -667,15 +669,10 @@ static hipError_t launch_k(const LmHeadArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// 64 columns a workgroup until 128 would fill the chip's CUs once.
-// k_lmhead up to kWideRows rows. Both sides, microseconds at D = 1280, V = 8194
-// (bf16 / fp32 / 8-bit): 128 rows 27.1 / 30.1 / 32.1 there, 29.0 / 29.1 / 31.0 here;
-// 256 rows 40.4 / 47.4 / 51.1 there, 38.0 / 38.2 / 39.9 here (rows up to 256 cost
-// the same here, each 64 rows a pass there).
-constexpr int kWideRows = 192;
 template <int WK>
 static hipError_t launch_wide(const LmHeadArgs& a, hipStream_t s) {
   const int mt = (a.M + kWdM - 1) / kWdM;
+  // 64 columns a workgroup until 128 would fill the chip's CUs once
   if ((int64_t)mt * ((a.V + 127) / 128) >= 256)
     hipLaunchKernelGGL((k_lmhead_wide<WK, 128>), dim3((a.V + 127) / 128, mt), dim3(kWdThreads), 0, s, a);
   else
@@ -683,8 +680,27 @@ static hipError_t launch_wide(const LmHeadArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Whether k_lmhead_wide takes a call. Up to kWideRows rows k_lmhead does (128
+// rows of 1280 x 8194, bf16 / fp32 / 8-bit: 27 / 30 / 30 us there, 30 / 29 / 32
+// here; 256 rows 41 / 47 / 46 there, 38 / 38 / 39 here), and wherever its tiles,
+// two a CU, go in one round: a wide workgroup alone on its CU takes about twice
+// as long as that round (1000 rows of 1280 x 500: 13 / 14 / 15 us there, 29 / 28
+// / 33 here; 256 of 1280 x 2000: 13 / 16 / 15 and 29 / 28 / 33). In the second
+// round bf16 weights, which need the least conversion, still do better there
+// unless K is short (1280 inputs, 768 tiles: 28 us and 34; 1028 tiles 41 and 38;
+// 256 inputs, 564 tiles: 14 and 11), fp32 and most 8-bit ones do not (1280
+// inputs, 630 tiles: fp32 35 and 28, 8-bit 34 and 33; 1792 inputs, 8-bit, up to
+// 768 tiles, 8% for k_lmhead).
+constexpr int kWideRows = 192;
+constexpr int kLmRound = 512;   // k_lmhead's tiles of one round
+static bool lmhead_wide_pays(const LmHeadArgs& a) {
+  const int64_t tiles = (int64_t)((a.V + kTileN - 1) / kTileN) * ((a.M + 63) / 64);
+  const int64_t most = a.wkind == kLmW_BF16 ? std::min(std::max(a.D, kLmRound), 2 * kLmRound) : kLmRound;
+  return a.M > kWideRows && tiles > most;
+}
+
 hipError_t launch_lmhead(const LmHeadArgs& a, hipStream_t s) {
-  if (a.M > kWideRows) {
+  if (lmhead_wide_pays(a)) {
     switch (a.wkind) {
       case kLmW_BF16: return launch_wide<kLmW_BF16>(a, s);
       case kLmW_F32: return launch_wide<kLmW_F32>(a, s);

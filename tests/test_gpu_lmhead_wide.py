@@ -1,5 +1,6 @@
-"""LM head at the edges of its tiles' row counts (16, 32, 64 and, past 192, 128
-rows with 64 or 128 columns and chunks of 64 inputs), for the three weight kinds,
+"""LM head at the edges of its tiles' row counts (16, 32, 64 and, past 192 rows and
+a round of those tiles, 128 rows with 64 or 128 columns and chunks of 64 inputs),
+for the three weight kinds,
 against the float64 oracle; the tolerance and its derivation are test_gpu_lmhead's (the same split
 of the weights, the same sums)."""
 import numpy as np
@@ -18,7 +19,13 @@ CASES = [("bf16", 1, 1280, 8194, 64, 0.0), ("f32", 1, 320, 33, 32, 4.0), ("q8", 
          ("bf16", 257, 160, 65, 32, 4.0), ("bf16", 192, 160, 65, 32, 0.0), ("bf16", 300, 1280, 8194, 64, 0.0), ("bf16", 777, 1280, 5000, 64, 0.0),
          ("f32", 193, 96, 129, 32, 0.0), ("f32", 200, 2080, 127, 32, 4.0), ("f32", 520, 256, 8194, 64, 0.0),
          ("q8", 194, 32, 40, 32, 0.0), ("q8", 230, 192, 65, 64, 0.0), ("q8", 257, 256, 130, 128, 4.0),
-         ("q8", 600, 1280, 8194, 64, 0.0), ("q8", 1000, 96, 4100, 32, 0.0)]
+         ("q8", 600, 1280, 8194, 64, 0.0), ("q8", 1000, 96, 4100, 32, 0.0),
+         # past a round of the smaller tiles (512 of 32 columns x 64 rows; bf16 up to 1024 of long K)
+         ("bf16", 193, 32, 4096, 32, 0.0), ("bf16", 193, 32, 4097, 32, 0.0), ("bf16", 255, 96, 4159, 32, 0.0),
+         ("bf16", 256, 64, 4160, 32, 0.0), ("bf16", 257, 160, 4161, 32, 4.0), ("bf16", 200, 1024, 8193, 64, 0.0),
+         ("bf16", 200, 1024, 8192, 64, 0.0), ("f32", 193, 96, 4223, 32, 0.0), ("f32", 200, 224, 4225, 32, 4.0),
+         ("f32", 1030, 32, 961, 32, 0.0), ("q8", 194, 32, 4104, 32, 0.0), ("q8", 230, 192, 4161, 64, 0.0),
+         ("q8", 257, 256, 4099, 128, 4.0)]
 
 
 @pytest.mark.parametrize("kind,M,D,V,group,shift", CASES)
