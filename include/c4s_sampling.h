@@ -24,16 +24,17 @@
  *     owns every input/output buffer (device memory); the context owns its
  *     workspace. A context is not thread-safe: use one per host thread.
  *   - Workspaces grow on first use (hipMalloc, which synchronises the device).
- *     c4s_sample_rows with vocab <= 12288 uses none. While the stream is being
- *     captured into a graph a workspace never grows (C4S_EINVAL): make one call
- *     of the same shape outside the capture first. Once a captured call used a
- *     workspace, a later growth keeps the old buffer alive until c4s_destroy.
- *     Rows with vocab > 12288 have a workspace per stream (for up to eight
- *     streams; a further one waits for the device and takes over the one used
- *     longest ago), so such calls of one context may be in flight on several
- *     streams. A graph's replays use the workspace its capture took (its
- *     stream's, or another stream's that is large enough): the caller orders
- *     them with other large-vocabulary calls that may share it.
+ *     c4s_sample_rows with vocab <= 12288 uses none. c4s_sample_rows at larger
+ *     vocabularies, and c4s_lmhead_sample (its logits, when the caller gives no
+ *     buffer), have a workspace per stream, so such calls of one context may be
+ *     in flight on several streams. Eight streams have one each; a further one
+ *     takes over the one used longest ago and waits for its last call on the
+ *     device.
+ *   - Under capture into a graph a call is taken when an earlier call of the
+ *     context outside a capture was of the same size or larger, else it is
+ *     C4S_EINVAL. It then gets a workspace that no call outside a capture uses,
+ *     kept until c4s_destroy. Graphs captured on one stream share it: replays of
+ *     them must not overlap each other; they may overlap any other call.
  *   - Input contract: logits are finite or -inf (no +inf/NaN), temperature is
  *     1, <= 0, or keeps logits/temperature finite.
  *   - top_p tie order: when the nucleus cut falls inside a group of equal

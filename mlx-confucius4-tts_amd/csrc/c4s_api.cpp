@@ -14,13 +14,31 @@
 
 #include "../../include/c4s_sampling.h"
 #include "c4s_internal.h"
+#include "c4s_pool.hpp"
 
-// Workspace of the large-vocabulary rows of one stream.
-struct RowsWs {
-  hipStream_t stream = nullptr;
-  void* p = nullptr;
-  size_t bytes = 0;
-  uint64_t used = 0;   // tick of its last call
+// The pools' runtime.
+struct HipRt {
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  hipError_t err = hipSuccess;   // of the last call
+  bool ok(hipError_t e) {
+    err = e;
+    return e == hipSuccess;
+  }
+  // While any stream of the thread is being captured, hipMalloc is refused
+  // (and the capture lost) unless the thread asks for the relaxed mode.
+  bool alloc(void** p, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (!ok(hipThreadExchangeStreamCaptureMode(&mode))) return false;
+    const hipError_t e = hipMalloc(p, bytes);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok(e);
+  }
+  bool release(void* p) { return ok(hipFree(p)); }
+  bool create(hipEvent_t* e) { return ok(hipEventCreateWithFlags(e, hipEventDisableTiming)); }
+  bool destroy(hipEvent_t e) { return ok(hipEventDestroy(e)); }
+  bool record(hipEvent_t e, hipStream_t s) { return ok(hipEventRecord(e, s)); }
+  bool wait(hipStream_t s, hipEvent_t e) { return ok(hipStreamWaitEvent(s, e, 0)); }
 };
 
 struct c4s_ctx {
@@ -29,14 +47,8 @@ struct c4s_ctx {
   hipStream_t host_stream = nullptr;  // used by the synchronous host helpers
   void* ws = nullptr;                 // stream: exact steps' key buffers
   size_t ws_bytes = 0;
-  // Large-vocabulary rows (slices, lists, exact-pass keys): one per stream that
-  // issues such calls, so that calls on several streams do not share one.
-  static constexpr int kRowsWs = 8;
-  RowsWs rows_ws[kRowsWs];
-  int n_rows_ws = 0;
-  uint64_t rows_tick = 0;
-  void* logits_ws = nullptr;          // LM head + sample: logits when the caller gives none
-  size_t logits_bytes = 0;
+  c4s::StreamPool<HipRt> rows_ws;     // large-vocabulary rows: slices, lists, exact-pass keys
+  c4s::StreamPool<HipRt> logits_ws;   // LM head + sample: logits when the caller gives none
   // host-helper staging: pinned host memory that the device maps
   void* hstage = nullptr;
   size_t hstage_bytes = 0;
@@ -62,11 +74,6 @@ struct c4s_ctx {
   // step segments of the pipelined row chain (rows without penalty)
   void* segres = nullptr;
   size_t segres_bytes = 0;
-  // Set once a call on a capturing stream used a workspace: from then on a
-  // workspace that grows is retired (freed at c4s_destroy) instead of freed,
-  // because a captured graph may still write the old buffer when replayed.
-  bool graph_used = false;
-  std::vector<void*> retired;
   // this device's address of the no-allocation entry point's static scratch
   // (null when the runtime could not give it)
   void* noalloc = nullptr;
@@ -132,30 +139,14 @@ bool is_capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
 }
 
-// Workspace of at least `need` bytes for a call queued on `s`. A workspace
-// never grows while `s` is being captured into a graph (allocation is not
-// allowed there): a first call of the same shape outside the capture sizes it.
-int ensure(c4s_ctx* ctx, void** buf, size_t* have, size_t need, const char* what, hipStream_t s) {
-  const bool cap = is_capturing(s);
-  if (need <= *have) {
-    if (cap) ctx->graph_used = true;
-    return C4S_OK;
-  }
-  if (cap)
-    return fail(ctx, C4S_EINVAL, std::string(what) +
-                                     ": the workspace would grow during graph capture; make one call of "
-                                     "this shape (or larger) outside the capture first");
+// Workspace of at least `need` bytes for a sample_stream call (which is never captured).
+int ensure(c4s_ctx* ctx, void** buf, size_t* have, size_t need, const char* what) {
+  if (need <= *have) return C4S_OK;
   if (*buf) {
-    if (ctx->graph_used) {   // a graph may still use it: keep it until c4s_destroy
-      ctx->retired.push_back(*buf);
-      *buf = nullptr;
-      *have = 0;
-    } else {
-      hipError_t e = hipFree(*buf);
-      *buf = nullptr;
-      *have = 0;
-      if (e != hipSuccess) return hip_fail(ctx, e, what);
-    }
+    hipError_t e = hipFree(*buf);
+    *buf = nullptr;
+    *have = 0;
+    if (e != hipSuccess) return hip_fail(ctx, e, what);
   }
   hipError_t e = hipMalloc(buf, need);
   if (e != hipSuccess) {
@@ -165,6 +156,21 @@ int ensure(c4s_ctx* ctx, void** buf, size_t* have, size_t need, const char* what
   }
   *have = need;
   return C4S_OK;
+}
+
+// The stream's workspace of `pool` for a call about to be queued on `s`.
+int pool_take(c4s_ctx* ctx, c4s::StreamPool<HipRt>& pool, hipStream_t s, size_t need, const char* what, void** out) {
+  switch (pool.take(s, is_capturing(s), need, out)) {
+    case c4s::PoolResult::kOk: return C4S_OK;
+    case c4s::PoolResult::kWouldGrow:
+      return fail(ctx, C4S_EINVAL, std::string(what) +
+                                       ": the workspace would grow during graph capture; make one call of "
+                                       "this shape (or larger) outside the capture first");
+    default: break;
+  }
+  const hipError_t e = pool.runtime().err;
+  return e == hipErrorOutOfMemory ? fail(ctx, C4S_ENOMEM, std::string(what) + ": out of memory")
+                                  : hip_fail(ctx, e, what);
 }
 
 size_t pow2_at_least(size_t n) {
@@ -234,59 +240,30 @@ c4s::RowsArgs to_args(const c4s_rows* r) {
 }
 
 // The workspace of vocabularies the step cannot stage in LDS, for a call queued
-// on `s` (*out: null below that size). A captured call takes its stream's, or
-// another stream's that is large enough (a graph's replays are ordered by the
-// caller), and never allocates. Past kRowsWs streams the one used longest ago
-// is handed on once the device is idle.
+// on `s` (*out: null below that size).
 int rows_workspace(c4s_ctx* ctx, const c4s_rows* r, hipStream_t s, void** out) {
   *out = nullptr;
   if (r->vocab <= c4s::kLdsVocabMax) return C4S_OK;
   const size_t need = pow2_at_least((size_t)r->vocab) * sizeof(uint32_t) * (size_t)r->n_rows;
-  RowsWs* w = nullptr;
-  for (int i = 0; i < ctx->n_rows_ws; ++i)
-    if (ctx->rows_ws[i].stream == s) w = &ctx->rows_ws[i];
-  if (is_capturing(s)) {
-    for (int i = 0; i < ctx->n_rows_ws && (!w || w->bytes < need); ++i)
-      if (ctx->rows_ws[i].bytes >= need) w = &ctx->rows_ws[i];
-    if (!w || w->bytes < need)
-      return fail(ctx, C4S_EINVAL, "sort workspace: the workspace would grow during graph capture; make one call of "
-                                   "this shape (or larger) outside the capture first");
-    ctx->graph_used = true;
-  } else {
-    if (!w && ctx->n_rows_ws < c4s_ctx::kRowsWs) {
-      w = &ctx->rows_ws[ctx->n_rows_ws++];
-      w->stream = s;
-    } else if (!w) {
-      w = &ctx->rows_ws[0];
-      for (RowsWs& o : ctx->rows_ws)
-        if (o.used < w->used) w = &o;
-      const hipError_t e = hipDeviceSynchronize();
-      if (e != hipSuccess) return hip_fail(ctx, e, "sort workspace");
-      w->stream = s;
-    }
-    if (w->bytes < need) {
-      const int rc = ensure(ctx, &w->p, &w->bytes, need, "sort workspace", s);
-      if (rc) return rc;
-    }
-  }
-  w->used = ++ctx->rows_tick;
-  *out = w->p;
+  return pool_take(ctx, ctx->rows_ws, s, need, "sort workspace", out);
+}
+
+// The rows on workspace `ws` (rows_workspace).
+int launch_rows_on(c4s_ctx* ctx, const c4s_rows* r, void* ws, hipStream_t s) {
+  c4s::RowsArgs a = to_args(r);
+  a.sort_ws = static_cast<uint32_t*>(ws);
+  a.sort_ws_stride = ws ? (int64_t)pow2_at_least((size_t)r->vocab) : 0;
+  hipError_t e = c4s::launch_rows(a, s);
+  if (ws) ctx->rows_ws.queued(s, is_capturing(s));
+  if (e != hipSuccess) return hip_fail(ctx, e, "sample_rows launch");
   return C4S_OK;
 }
 
 int launch_rows_checked(c4s_ctx* ctx, const c4s_rows* r, hipStream_t s) {
-  c4s::RowsArgs a = to_args(r);
-  if (r->vocab > c4s::kLdsVocabMax) {
-    const size_t per_row = pow2_at_least((size_t)r->vocab) * sizeof(uint32_t);
-    void* ws = nullptr;
-    int rc = rows_workspace(ctx, r, s, &ws);
-    if (rc) return rc;
-    a.sort_ws = static_cast<uint32_t*>(ws);
-    a.sort_ws_stride = (int64_t)(per_row / sizeof(uint32_t));
-  }
-  hipError_t e = c4s::launch_rows(a, s);
-  if (e != hipSuccess) return hip_fail(ctx, e, "sample_rows launch");
-  return C4S_OK;
+  void* ws = nullptr;
+  int rc = rows_workspace(ctx, r, s, &ws);
+  if (rc) return rc;
+  return launch_rows_on(ctx, r, ws, s);
 }
 
 }  // namespace
@@ -359,11 +336,10 @@ int c4s_destroy(c4s_ctx* ctx) {
   if (ctx->scan_s) (void)hipStreamSynchronize(ctx->scan_s);
   for (hipStream_t st : {ctx->scan_m, ctx->chain_m, ctx->side_m})
     if (st) (void)hipStreamSynchronize(st);
-  for (void* p : {ctx->ws, ctx->logits_ws, ctx->sum_ws, ctx->state_ws, ctx->segres})
+  for (void* p : {ctx->ws, ctx->sum_ws, ctx->state_ws, ctx->segres})
     if (p) (void)hipFree(p);
-  for (const RowsWs& w : ctx->rows_ws)
-    if (w.p) (void)hipFree(w.p);
-  for (void* p : ctx->retired) (void)hipFree(p);
+  ctx->rows_ws.clear();
+  ctx->logits_ws.clear();
   if (ctx->host_stream) (void)hipStreamDestroy(ctx->host_stream);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   if (ctx->scan_s) (void)hipStreamDestroy(ctx->scan_s);
@@ -550,20 +526,20 @@ int c4s_sample_stream(c4s_ctx* ctx, const c4s_stream* st, void* stream) {
   const int chunk = (int)std::max<size_t>(1, chunk_sz);   // the longest chunk
   const size_t chunk_bytes = per_step * (size_t)chunk;
   const int n_bufs = chunk >= a.n_steps ? 1 : overlap ? kOverlapBufs : 2;
-  int rc = ensure(ctx, &ctx->sum_ws, &ctx->sum_bytes, (size_t)n_bufs * chunk_bytes, "stream summaries", hs);
+  int rc = ensure(ctx, &ctx->sum_ws, &ctx->sum_bytes, (size_t)n_bufs * chunk_bytes, "stream summaries");
   if (rc) return rc;
-  rc = ensure(ctx, &ctx->state_ws, &ctx->state_bytes, (size_t)a.n_rows * c4s::kStateWords * 4, "stream state", hs);
+  rc = ensure(ctx, &ctx->state_ws, &ctx->state_bytes, (size_t)a.n_rows * c4s::kStateWords * 4, "stream state");
   if (rc) return rc;
   // The chains' exact steps sort in a per-row global key buffer.
   const size_t sort_row = pow2_at_least((size_t)a.vocab) * sizeof(uint32_t);
-  rc = ensure(ctx, &ctx->ws, &ctx->ws_bytes, sort_row * (size_t)a.n_rows, "sort workspace", hs);
+  rc = ensure(ctx, &ctx->ws, &ctx->ws_bytes, sort_row * (size_t)a.n_rows, "sort workspace");
   if (rc) return rc;
   // Rows without penalty split their steps into segments, one workgroup each,
   // over the CUs the chains have (every workgroup of the pipelined chain
   // holds a CU's LDS).
   const int nseg = std::max(2, std::min(kMaxSegments, (overlap ? row_cus(ctx) : ctx->n_cus) / std::max(1, a.n_rows)));
   rc = ensure(ctx, &ctx->segres, &ctx->segres_bytes, (size_t)a.n_rows * nseg * 4 * sizeof(uint64_t),
-              "segment results", hs);
+              "segment results");
   if (rc) return rc;
   // Full-vocabulary rows: the speculative chain (several steps decided at
   // once, each checked in order) when a call's drawn ids fit its lists, else
@@ -735,20 +711,20 @@ int c4s_lmhead_sample(c4s_ctx* ctx, const c4s_head* head, const c4s_rows* rows, 
   DeviceGuard g(ctx->device);
   if (g.err != hipSuccess) return hip_fail(ctx, g.err, "hipSetDevice");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  float* logits = head->logits;
-  if (!logits) {
-    rc = ensure(ctx, &ctx->logits_ws, &ctx->logits_bytes,
-                (size_t)std::max(head->M, 1) * (size_t)std::max(head->V, 1) * 4, "logits workspace", s);
+  void* lws = nullptr;
+  if (!head->logits) {
+    rc = pool_take(ctx, ctx->logits_ws, s, (size_t)std::max(head->M, 1) * (size_t)std::max(head->V, 1) * 4,
+                   "logits workspace", &lws);
     if (rc) return rc;
-    logits = static_cast<float*>(ctx->logits_ws);
-    r.logits = logits;
+    r.logits = lws;
   }
   void* ws = nullptr;
   rc = rows_workspace(ctx, &r, s, &ws);
   if (rc) return rc;
-  rc = lmhead_launch(ctx, head, logits, r.ld, s);
-  if (rc) return rc;
-  return launch_rows_checked(ctx, &r, s);
+  rc = lmhead_launch(ctx, head, head->logits ? head->logits : static_cast<float*>(lws), r.ld, s);
+  if (!rc) rc = launch_rows_on(ctx, &r, ws, s);
+  if (lws) ctx->logits_ws.queued(s, is_capturing(s));
+  return rc;
 }
 
 int c4s_lmhead_sample_noalloc(c4s_ctx* ctx, const c4s_head* head, const c4s_rows* rows, void* stream) {
