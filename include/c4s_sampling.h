@@ -37,6 +37,13 @@
  *     them must not overlap each other; they may overlap any other call.
  *   - Input contract: logits are finite or -inf (no +inf/NaN), temperature is
  *     1, <= 0, or keeps logits/temperature finite.
+ *   - Not determined: top_p 0 (or so small that 1 - top_p is 1 to within the
+ *     rounding of the sums) with min_keep 0. The reference then removes every id
+ *     whose sum of quotients is at most 1, and whether the last sum, over all of
+ *     them, rounds above 1 depends on the last bit of the host's exp. Such a row
+ *     keeps its largest value or nothing (id 0 is drawn); in 1 to 3 rows of 100
+ *     it is not what a host with glibc gives. min_keep 1, the reference's
+ *     default, keeps the largest value in either case.
  *   - top_p tie order: when the nucleus cut falls inside a group of equal
  *     values, the lower token ids of that group survive. (The reference's
  *     unstable std::sort leaves this choice to the host's sort permutation.)
