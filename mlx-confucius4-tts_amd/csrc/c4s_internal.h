@@ -140,6 +140,7 @@ size_t rows_global_lds_bytes(int vocab);
 size_t stream_lds_bytes(int vocab, int unused);
 
 hipError_t launch_rows(const RowsArgs& a, hipStream_t s);
+hipError_t launch_rows_step(const RowsArgs& a, hipStream_t s);   // vocabularies that fit LDS
 bool rows_step_many_fits(const RowsArgs& a);   // the one-pass step in the form that shares a CU
 hipError_t launch_rows_step_many(const RowsArgs& a, hipStream_t s);
 hipError_t launch_hist_bits_init(const int32_t* ids, const int64_t* off, int n_rows, int V, uint32_t* bits,

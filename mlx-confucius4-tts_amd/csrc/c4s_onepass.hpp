@@ -329,7 +329,7 @@ __device__ __noinline__ int tie_cut(const RowCfg& c, const float* val, int lo, i
 // The multi-pass chain (c4s_chain.hpp) on the penalised row staged in LDS
 // (`val`), for the rows the one pass leaves; kept out of line so that its
 // registers do not weigh on the one-pass path.
-__device__ __noinline__ void chain_fallback(const StepIO& io, const RowCfg& c, unsigned char* work, float* val,
+[[maybe_unused]] __device__ __noinline__ void chain_fallback(const StepIO& io, const RowCfg& c, unsigned char* work, float* val,
                                             StepScratch& sh, bool tp_exact_first) {
   const int V = c.V, t = threadIdx.x;
   uint64_t rng = *io.rng;
@@ -966,20 +966,6 @@ __device__ __forceinline__ bool sampled_step(const StepIO& io, const RowCfg& c, 
     }
   }
   return false;
-}
-
-// One AR step of the reference chain (C4S_MODE_CHAIN) for one row per
-// workgroup, in one pass where it can (c4s_step.hpp), else the multi-pass
-// chain on the row staged in LDS. PT >= the ids a thread owns.
-// Byte i of a per-row flag array, nonzero or not, read through the aligned
-// dword that holds it: a scalar load (the flags are the same for the whole
-// workgroup), where a byte load would go through the vector memory path and be
-// waited for at once. The dword never leaves the allocation's 256-byte granule.
-__device__ __forceinline__ bool flag_byte(const uint8_t* __restrict__ p, int i) {
-  const uint8_t* b = p + i;
-  const int sh = (int)(reinterpret_cast<uintptr_t>(b) & 3);
-  const uint32_t wd = *reinterpret_cast<const uint32_t*>(b - sh);
-  return ((wd >> (8 * sh)) & 0xFFu) != 0u;
 }
 
 }  // namespace

@@ -199,7 +199,7 @@ struct Boundary {
   double mabove;    // their mass
   uint32_t thru;    // entries up to and including bucket hi
 };
-__device__ Boundary boundary_scan(const uint32_t* cnt, const double* ms, bool topk, uint32_t k, double Blo,
+[[maybe_unused]] __device__ Boundary boundary_scan(const uint32_t* cnt, const double* ms, bool topk, uint32_t k, double Blo,
                                   double Bhi, uint32_t c0, double m0) {
   const int lane = lane_id();
   uint32_t c4[4], lc = 0;
@@ -439,7 +439,7 @@ __device__ __forceinline__ float kept_mass32(const KeptRule& kr, float z, float 
 // first id whose prefix reaches r = u * sum taken when both ends of its
 // interval are farther than rel_eps from r; otherwise the reference's
 // sequential sums in id order.
-__device__ __noinline__ int draw_replay(const StepIO& io, const RowCfg& c, const KeptRule kr, float m, double u) {
+[[maybe_unused]] __device__ __noinline__ int draw_replay(const StepIO& io, const RowCfg& c, const KeptRule kr, float m, double u) {
   const int lane = lane_id();
   const int V = c.V;
   auto mass_at = [&](int i) -> double {
@@ -595,6 +595,17 @@ __device__ __forceinline__ float* stage_row_bf16(const uint16_t* p, int V, float
   }
   if (eidx >= 0) val[eidx] = __uint_as_float((uint32_t)ev << 16);
   return val;
+}
+
+// Byte i of a per-row flag array, nonzero or not, read through the aligned
+// dword that holds it: a scalar load (the flags are the same for the whole
+// workgroup), where a byte load would go through the vector memory path and be
+// waited for at once. The dword never leaves the allocation's 256-byte granule.
+__device__ __forceinline__ bool flag_byte(const uint8_t* __restrict__ p, int i) {
+  const uint8_t* b = p + i;
+  const int sh = (int)(reinterpret_cast<uintptr_t>(b) & 3);
+  const uint32_t wd = *reinterpret_cast<const uint32_t*>(b - sh);
+  return ((wd >> (8 * sh)) & 0xFFu) != 0u;
 }
 
 }  // namespace
