@@ -193,9 +193,10 @@ __device__ __forceinline__ uint64_t xor_lane_u64(uint64_t v) {
 // One multiply and two conversions instead of the IEEE divide's ten steps.
 __device__ __forceinline__ float div_rcp(float x, double r) { return (float)((double)x * r); }
 
-// exp(t) for t <= 0 (-inf gives 0) to about an ulp: 2^n e^r, |r| <= ln 2 / 2,
-// e^r by its Taylor polynomial of degree 12 (the first term left out is below
-// 2^-52 e^r); rel_eps covers a few ulp.
+// exp(t) for t <= 0 (-inf gives 0) to about an ulp: 2^n e^r, |r| <= ln 2 / 2, r by
+// Cody and Waite's reduction (ln 2 in two parts, n times the first exact), e^r by
+// its Taylor polynomial of degree 12 (what it leaves out is at most 1.04 x 2^-52
+// e^r, at r = -ln 2 / 2); rel_eps covers a few ulp.
 __device__ __forceinline__ double exp_neg(double t) {
   t = fmax(t, -746.0);   // 0 from there on
   const double n = rint(t * 0x1.71547652b82fep+0);
