@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
 // split). 8-bit codes are taken to scale q + offset in fp32 first, so that no
 // per-group partial products are needed. Loads run one chunk ahead in registers;
 // two workgroups share a CU, so one converts while the other multiplies. 777
-// rows: 59 us bf16, 64 fp32, 63 8-bit (k_lmhead 100, 121, 133); a thread's
+// rows: 58.5 us bf16, 63.5 fp32, 62.3 8-bit (k_lmhead 100, 121, 133); a thread's
 // weights as 32 inputs of one column (64 bytes a lane: eight lanes' loads on one
 // line before) 64 / 104 / 65, and gamma and beta loaded by the threads that
 // convert 72 / 102 / 75.
@@ -415,8 +415,8 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
 // eighth, joined in double. As one fp32 sum over D each (and d + bias in fp32)
 // rows offset by 16 sigma were off by 4.8e-5 (D = 1280) and 6.1e-5 (D = 4096)
 // of the logits, now 3.9e-5 and 4.6e-5; k_lmhead 3.9e-5 and 4.5e-5. A quarter
-// ends where no load of a chunk is in flight: at the end of the loop body
-// instead, 73 us bf16; as a loop around the chunks, 60. G's own sum runs over
+// ends between the barrier and the products: behind the products instead, 73 us
+// bf16; as a loop around the chunks, 60; before the next chunk's loads, 58.9. G's own sum runs over
 // all of D in the accumulators (k_lmhead: four, joined in fp32), which is 0.5%
 // of the error at D = 1280 and 2% at 4096; a second set of accumulators beside
 // the first does not fit the registers (74 us).
@@ -434,6 +434,7 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
   __shared__ __align__(16) unsigned char xs[kWdM * kWdPitch], wh[BN * kWdPitch], wl[BN * kWdPitch];
   __shared__ __align__(16) float gb[2][2][kWdK];   // by buffer: gamma, beta of a chunk
   __shared__ float st1[4][kWdM], st2[4][kWdM];   // by quarter of D: a row's sums of x and of x^2
+  __shared__ __align__(16) float cpart[BN][8], dpart[BN][8];   // by thread: a column's c and d
   __shared__ float rmu[kWdM], rinv[kWdM], ccol[BN], dcol[BN];
   const int D = a.D, V = a.V, M = a.M;
   const int n0 = blockIdx.x * BN, m0 = blockIdx.y * kWdM;
@@ -547,9 +548,9 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
         *reinterpret_cast<uint4*>(&wl[(kRows * j + pr) * kWdPitch + pk * 2]) = lo;
       }
     }
-    if (ch == nq * (q + 1)) keep();   // with no load of a chunk in flight
     if (ch + 1 < nch) fetch(ch + 1);   // in flight during the products
     __syncthreads();
+    if (ch == nq * (q + 1)) keep();
 #pragma unroll
     for (int ks = 0; ks < kWdK / 32; ++ks) {
       const int ko = ks * 64 + g * 16;   // bytes: 32 inputs a step, 8 a lane group
@@ -577,20 +578,13 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
   keep();
 #pragma unroll
   for (int j = 0; j < kWp; ++j) {   // eight threads hold a column's inputs
-    double cc = (double)cp[j], dd = (double)dp[j];
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) {
-      cc += __shfl_xor(cc, o, kWave);
-      dd += __shfl_xor(dd, o, kWave);
-    }
-    if (t % 8 == 0) {
-      const int cl = kRows * j + pr;
-      ccol[cl] = (float)cc;
-      dcol[cl] = (float)(dd + (double)a.bias[min(n0 + cl, V - 1)]);
-    }
+    cpart[kRows * j + pr][t % 8] = cp[j];
+    dpart[kRows * j + pr][t % 8] = dp[j];
   }
+  const int cl = t - kWdM;   // the upper threads' column, the lower ones' row t
+  const float bias = cl >= 0 && cl < BN ? a.bias[min(n0 + cl, V - 1)] : 0.f;
   __syncthreads();
-  if (t < kWdM) {
+  if (cl < 0) {
     const double invD = 1.0 / (double)D;
     double S1 = 0.0, S2 = 0.0;
     for (int i = 0; i < q; ++i) {   // the quarters that D has
@@ -600,6 +594,15 @@ __global__ __launch_bounds__(kWdThreads) __attribute__((amdgpu_waves_per_eu(2)))
     const double mu = S1 * invD;
     rmu[t] = (float)mu;
     rinv[t] = (float)(1.0 / sqrt(fmax(S2 * invD - mu * mu, 0.0) + (double)a.eps));
+  } else if (cl < BN) {
+    double cc = 0.0, dd = (double)bias;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      cc += (double)cpart[cl][i];
+      dd += (double)dpart[cl][i];
+    }
+    ccol[cl] = (float)cc;
+    dcol[cl] = (float)dd;
   }
   __syncthreads();
 #pragma unroll
