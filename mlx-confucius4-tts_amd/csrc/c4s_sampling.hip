@@ -861,7 +861,10 @@ constexpr int kBigThreads = 512;   // phases A and B by slices
 // workgroups pass the CUs; bf16, 32 rows 24 / 52 / 15 against 77 / 160 / 35, 256
 // rows 68 / 159 / 40 against 79 / 164 / 36. At V = 20000 (2 slices) the
 // launches cost more than spreading gives: 64 fp32 rows 20 / 35 / 14 against
-// 13 / 45 / 11.
+// 13 / 45 / 11. The host does not see the rows' parameters, so the fp32 line is
+// the top-k rows', and nucleus and greedy rows beyond it pay for that: 64 rows of
+// 151936 as above, 50257 ids (4 slices) 17 / 74 / 18 in one workgroup a row where
+// bf16 rows by phases take 22 / 38 / 14.
 bool big_by_phase(const RowsArgs& a) {
   const int nsl = big_slices(a.vocab);
   return a.dtype == 0 ? nsl >= 8 && (int64_t)nsl * a.n_rows <= 320 : nsl >= 4;
