@@ -150,9 +150,10 @@ __global__ __launch_bounds__(kLmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   // complete in issue order, so a chunk's rows of x, issued two chunks ahead,
   // wait behind every weight load issued before them: a window of two chunks
   // (refilled per chunk) instead of the whole of K for bf16 weights took
-  // 64 x 1280 x 8194 from 15.7 to 13.8 us; 1 row, fp32: one chunk 11.45, two 11.6,
-  // all five 13.3 us.
-  constexpr int kWin = MT < 4 ? (kQ ? 2 : 1) : WK == kLmW_F32 ? 2 : (WK == kLmW_Q8 ? (SPU > 1 ? 2 : 3) : 2);
+  // 64 x 1280 x 8194 from 15.7 to 13.8 us. 1 row, one chunk / two / all five: bf16
+  // 9.1 / 9.0 / - us on weights in the last-level cache, 17.2 / 16.0 / 17.7 on
+  // weights that are not; fp32 11.45 / 11.6 / 13.3 and 22.2 / 22.0 / 24.4.
+  constexpr int kWin = MT < 4 ? (WK == kLmW_F32 ? 1 : 2) : WK == kLmW_F32 ? 2 : (WK == kLmW_Q8 ? (SPU > 1 ? 2 : 3) : 2);
   __shared__ __align__(16) unsigned char xs[2 * kXBytes];
   __shared__ __align__(16) float gbs[2][2][kChunkK];   // by buffer: gamma, beta of the chunk
   // by buffer: gamma hi, gamma lo, beta hi, beta lo as bf16 (rows 0-3 of an MFMA
